@@ -67,6 +67,27 @@ __device__ __forceinline__ float mul_f16_rn(float x, uint32_t word) {
     return r;
 }
 
+// The Q8_0 fold without the int-to-float conversion.  A block's int32 sum P (|P| <= 32 * 128 * 128 = 2^19) comes out
+// of an MFMA whose accumulator starts at 2^19, so x = P + 2^19 is an integer of [0, 2^20], and read as fp32 those bits
+// are the denormal x 2^-149 exactly (fp32 spacing is uniform from zero up, which is what lets one power of two carry
+// the offset for both signs of P).  Then with sa' = sa 2^96 and sc = -sa 2^-34 (both exact scalings)
+//     fma(x 2^-149, sa', sc) = RN((x - 2^19) sa 2^-53) = RN(P sa) 2^-53
+// is the fold's first rounding, scaled by 2^-53, in one instruction instead of a conversion and a multiply.  The rest
+// of the fold runs in that scale (a power of two commutes with every rounding) and q8_unscale takes it off once, exactly.
+// Nothing under- or overflows differently while 2^-48 <= |sa| < 2^31 or sa = 0 (q8_scale_ok; a quantizer's scale is at
+// least 1e-10 / 127 > 2^-41): every nonzero |P sa sw| 2^-53 is then a normal fp32 (fp16 |sw| >= 2^-24), and an fp32 sum
+// of K / 32 <= 2^25 terms below 2^66 stays far from 2^128.  Zeros may differ in sign, which the running sum (never -0)
+// cannot show.  Rows outside the range take the plain fold.
+constexpr int kQ8Bias = 1 << 19;
+__device__ __forceinline__ bool q8_scale_ok(float sa) {
+    const uint32_t e = (__float_as_uint(sa) >> 23) & 0xff;               // zero, or 127 - 48 <= e < 127 + 31
+    return sa == 0.f || e - 79u < 79u;
+}
+__device__ __forceinline__ float q8_scale(float sa) { return __fmul_rn(sa, 0x1p96f); }
+__device__ __forceinline__ float q8_offset(float sa) { return __fmul_rn(sa, -0x1p-34f); }
+__device__ __forceinline__ float q8_unscale(float y) { return __fmul_rn(y, 0x1p53f); }
+__device__ __forceinline__ float q8_term(int x, float sas, float sac) { return __builtin_fmaf(__int_as_float(x), sas, sac); }
+
 // Every listed kernel argument in scalar registers at this point, with one wait: the compiler otherwise loads each
 // argument where it is first used, one scalar memory round trip after another, and a decode-size kernel's first
 // weight request then waits behind several of them.  Up to 16 arguments (all wave-uniform values).
@@ -170,13 +191,13 @@ __device__ __forceinline__ int wave_sum_width(int v, int width) {
     return v;
 }
 
-// Tile order for a grid of tiles_m x tiles_n output tiles: the hardware hands workgroup i to XCD i % 8, so logical
-// tile t = (i % 8) * (tiles / 8) + i / 8 gives each XCD a contiguous range of tiles, walked in groups of 8 tile-rows
-// (m fastest); the workgroups that run together on one XCD then share 8 m-tiles and 8 n-tiles through its L2.
+// Tile order for a grid of tiles_m x tiles_n output tiles: the hardware hands workgroup i to XCD i % 8, so giving XCD x the
+// logical tiles x (tiles / 8) + min(x, tiles % 8) + i / 8 (one more each for the first tiles % 8) puts a contiguous range
+// on each, walked in groups of 8 tile-rows (m fastest); the workgroups that run together on one XCD then share 8 m-tiles
+// and 8 n-tiles through its L2.
 __device__ __forceinline__ void xcd_tile_coords(int pid, int tiles_m, int tiles_n, int& pm, int& pn) {
-    const int total = tiles_m * tiles_n;
-    int t = pid;
-    if ((total & 7) == 0) t = (pid & 7) * (total >> 3) + (pid >> 3);
+    const int total = tiles_m * tiles_n, x = pid & 7;
+    const int t = x * (total >> 3) + min(x, total & 7) + (pid >> 3);
     constexpr int GM = 8;
     const int per_group = GM * tiles_n;
     const int first_m = (t / per_group) * GM;

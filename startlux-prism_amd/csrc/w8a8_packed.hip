@@ -13,6 +13,7 @@
 // Arithmetic: identical to the row-major kernels (kernels/w8a8.py:64-85), every output's fp32 sum over blocks in
 // block order, so both layouts give the same bits.
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "q8_stream.h"
@@ -246,12 +247,218 @@ constexpr int PBM = 128, PBN = 128;
 constexpr int PLDA = 128 + 16;          // activation tile row (bytes), padded
 constexpr int PLDB = 2048 + 64;         // one 16-row tile's two chunks, padded
 
+// The exact-order prefill tile: 128 x 32 NT outputs per 256-thread workgroup, each wave 32 activation rows x 32 NT columns
+// (NT v_mfma_i32_32x32x32_i8 per block), stages of 4 blocks (2 chunk pairs).  The VALU bounds it:
+// per output and block the fold is three instructions (q8_term, the weight scale's multiply, the add) beside 1/32 of an
+// MFMA.  One wave issues an independent VALU instruction every 4 clocks and a SIMD takes two waves' at once, so two waves
+// per SIMD fill it only if neither ever waits:
+//   * steps (block, column subtile) are software-pipelined through the whole K loop: step s + 1's MFMA and step s + 2's
+//     operand reads are issued before step s's fold, across stages too, and the fold runs as three groups of 16
+//     independent instructions (left to itself the compiler folds output by output, three dependent instructions
+//     behind an uncovered MFMA);
+//   * the weight stages are double-buffered in LDS: the next stage's registers are stored, and the one after requested,
+//     in the middle of a stage, with one barrier per stage, two steps before its end;
+//   * all of a wave's outputs lie on the same 32 rows: a lane holds the scaled activation scale and offset of 16 rows
+//     (32 registers; 64 if it held 64 x 64 outputs), and the activation fragments, which no other wave of an m-row
+//     needs, come straight from memory into the registers the MFMA reads, each block's a stage ahead.
+// Waves with no live row only stage the weights and keep the barriers.  PAN: `a` is the panel copy of
+// q8_act_panel_kernel, a fragment one 1 KB piece; otherwise it is 32 rows' 32 bytes.
+template <int EPI, bool PAN, int NT>
+__global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __restrict__ a,
+                                                                const float* __restrict__ a_s, int64_t as_sm,
+                                                                const int8_t* __restrict__ qt,
+                                                                const uint16_t* __restrict__ dt,
+                                                                void* __restrict__ out, int64_t ldo,
+                                                                const int32_t* __restrict__ n_rows, int M, int N,
+                                                                int K, int tiles_m, int tiles_n) {
+    constexpr int BN = 32 * NT, S = 4 * NT;
+    // one LDS buffer: the stage's 2 NT weight tiles (2 KB each), then its block scales.  ds_read_b128 serves 32 lanes in two
+    // groups, lanes 0-3, 12-15, 20-27 and the others; tiles at multiples of 256 bytes put each group on all 64 banks.
+    constexpr int OS = NT * 4096, BUF = OS + 4 * 128 * 4;
+    __shared__ __attribute__((aligned(16))) int8_t smem[2 * BUF];
+
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int pm, pn;
+    xcd_tile_coords(blockIdx.x, tiles_m, tiles_n, pm, pn);
+    const int m0 = pm * PBM, n0 = pn * BN;
+    const int live = min(M, __ldg(n_rows));
+    if (m0 >= live) return;
+    const int KP = K / 64, NS = K / 128;
+    const int nt0 = n0 / 16, ntiles = N / 16;
+
+    // Buffer loads, each operand's tile base in SGPRs and the stage's offset in soffset, so the loop computes no
+    // addresses; the record counts end with the operands, so rows past M or N read zeros.  Activations: lane l's 16
+    // bytes of a block are row l % 32, inputs 16 (l / 32) .. + 15.
+    const int mw = m0 + 32 * wv;                     // the wave's first row
+    const auto ar = PAN ? buf_rsrc(a + (int64_t)mw * K)
+                        : buf_rsrc_n(a + (int64_t)min(mw, M - 1) * K,
+                                     (uint32_t)min((int64_t)max(M - mw, 0) * K, (int64_t)0x7fffffff));
+    const uint32_t av = PAN ? lane * 16 : (lane & 31) * K + (lane >> 5) * 16;
+    // weights: chunk c = tid + 256 i -> tile c / 128, 16 bytes (c % 128) of its 2 KB run
+    const auto br = buf_rsrc_n(qt + (int64_t)nt0 * KP * 1024,
+                               (uint32_t)min((int64_t)(ntiles - nt0) * KP * 1024, (int64_t)0x7fffffff));
+    const uint32_t bv = (uint32_t)(tid >> 7) * KP * 1024 + (tid & 127) * 16;
+    // scales: thread -> tile tid / 32 (past the 2 NT: not read), pair (tid / 16) % 2, row tid % 16: both blocks' fp16
+    const auto sr = buf_rsrc_n(dt + (int64_t)nt0 * KP * 32,
+                               (uint32_t)min((int64_t)(ntiles - nt0) * KP * 64, (int64_t)0x7fffffff));
+    const uint32_t sv = (uint32_t)(tid >> 5) * KP * 64 + (tid & 31) * 4;
+
+    v4i rb[NT];
+    uint32_t rs;
+    auto gload = [&](int st) {                       // past the end: the last stage again
+        st = min(st, NS - 1);
+#pragma unroll
+        for (int i = 0; i < NT; i++) rb[i] = buf_load16<kBufNT>(br, bv, st * 2048 + i * 2 * KP * 1024);
+        rs = buf_load4(sr, sv, st * 128);
+    };
+    // A weight stage is stored block by block, [16-row tile][pair][block of the pair][q / 2][row][q % 2] of 8 bytes, so
+    // that a B fragment (below) is one 16-byte read, 16 lanes of it 256 contiguous bytes (no bank conflict).
+    int wb = (tid >> 7) * 2048 + ((tid >> 6) & 1) * 1024 + (lane >> 5) * 256 + (lane & 15) * 16 +
+             ((lane >> 4) & 1) * 8;
+    int ws = OS + ((tid >> 4) & 1) * 1024 + ((tid >> 5) * 16 + (tid & 15)) * 4;
+    int wflip = BUF;                                 // what takes the store addresses to the other buffer
+    auto store = [&]() {
+#pragma unroll
+        for (int i = 0; i < NT; i++) {
+            *reinterpret_cast<v2u*>(smem + wb + i * 4096) = v2u{(uint32_t)rb[i][0], (uint32_t)rb[i][1]};
+            *reinterpret_cast<v2u*>(smem + wb + i * 4096 + 512) = v2u{(uint32_t)rb[i][2], (uint32_t)rb[i][3]};
+        }
+        *reinterpret_cast<float*>(smem + ws) = f16_to_f32(rs & 0xffffu);
+        *reinterpret_cast<float*>(smem + ws + 512) = f16_to_f32(rs >> 16);
+        wb += wflip, ws += wflip, wflip = -wflip;
+    };
+
+    v4i fa[4];                                       // the wave's fragment of each block of a stage
+    auto load_a = [&](int st, int bi) {              // past the end: the last stage again
+        fa[bi] = buf_load16(ar, av, PAN ? min(st, NS - 1) * 4096 + bi * 1024 : min(st, NS - 1) * 128 + bi * 32);
+    };
+
+    const int lrow = 4 * (lane >> 5);
+    float sa[16], sc[16];
+    bool ok = true;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        sa[r] = a_s[(int64_t)min(mw + 8 * (r >> 2) + lrow + (r & 3), M - 1) * as_sm];
+        ok = ok && q8_scale_ok(sa[r]);
+    }
+    gload(0);
+    const bool all_ok = __syncthreads_and(ok);
+    load_a(0, 0);                                    // in the loop's own order, so that its waits can be as late
+    load_a(0, 1);
+    store();
+    gload(1);
+    load_a(0, 2);
+    load_a(0, 3);
+    lds_barrier();
+    if (mw >= live) {
+        for (int st = 0; st < NS; st++) {
+            store();
+            gload(st + 2);
+            lds_barrier();
+        }
+        return;
+    }
+
+    float y[NT][16];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) y[t][r] = 0.f;
+    // B fragment of column j = 32 t + lane % 32, lane group g = lane / 32: pieces q = 2 g, 2 g + 1 of row
+    // j % 16 in 16-row tile j / 16 (two tiles further per t)
+    const int swc = lane & 31;
+    int fbo = (swc >> 4) * 2048 + (lane >> 5) * 256 + (swc & 15) * 16;
+    int fso = OS + swc * 4, fflip = BUF;
+    auto loop = [&](auto plain) {
+        constexpr bool PLAIN = decltype(plain)::value;
+        v16i c0;
+#pragma unroll
+        for (int r = 0; r < 16; r++) c0[r] = PLAIN ? 0 : kQ8Bias;
+        if (!PLAIN) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) sc[r] = q8_offset(sa[r]), sa[r] = q8_scale(sa[r]);
+            asm volatile("" : "+v"(c0));             // held in registers, not made again before every MFMA
+        }
+        v4i fb[2];
+        v16i acc[2];
+        float sw[4];
+        auto frag = [&](int s) {                     // step s % S of the buffer the addresses point at
+            const int bi = s % S / NT, t = s % NT;
+            fb[s & 1] = *reinterpret_cast<const v4i*>(smem + fbo + t * 4096 + bi * 512);
+            if (t % 2 == 0) {                        // two subtiles' scales by one read
+                sw[s & 3] = *reinterpret_cast<const float*>(smem + fso + bi * 512 + t * 128);
+                if (t + 1 < NT) sw[(s + 1) & 3] = *reinterpret_cast<const float*>(smem + fso + bi * 512 + t * 128 + 128);
+            }
+        };
+        auto mfma = [&](int st, int s) {             // and, after a block's last MFMA, its registers' next block
+            const int bi = s % S / NT;
+            acc[s & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[bi], fb[s & 1], c0, 0, 0, 0);
+            if (s % NT == NT - 1) load_a(st + s / S + 1, bi);
+        };
+        frag(0);
+        frag(1);
+        mfma(0, 0);
+        for (int st = 0; st < NS; st++) {
+#pragma unroll
+            for (int s = 0; s < S; s++) {
+                if (s == S - 2) {                    // the next stage is in LDS, and this one's reads are done
+                    lds_barrier();
+                    fbo += fflip, fso += fflip, fflip = -fflip;
+                }
+                mfma(st, s + 1);
+                frag(s + 2);
+                if (s == S / 2 - 1) {
+                    store();
+                    gload(st + 2);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                float p[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    p[r] = PLAIN ? mul_rn((float)acc[s & 1][r], sa[r]) : q8_term(acc[s & 1][r], sa[r], sc[r]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int r = 0; r < 16; r++) p[r] = mul_rn(p[r], sw[s & 3]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int r = 0; r < 16; r++) y[s % NT][r] = add_rn(y[s % NT][r], p[r]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (!PLAIN) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) y[t][r] = q8_unscale(y[t][r]);
+        }
+    };
+    // every wave of the workgroup takes the same loop (the barriers are in it)
+    if (all_ok) loop(std::false_type{});
+    else loop(std::true_type{});
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int n = n0 + swc + 32 * t;
+        if (n >= N) continue;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int m = mw + 8 * (r >> 2) + lrow + (r & 3);
+            if (m < live) {
+                if (EPI == 0) {
+                    reinterpret_cast<uint16_t*>(out)[(int64_t)m * ldo + n] = (uint16_t)f32_to_bf16(y[t][r]);
+                } else {
+                    float* o = reinterpret_cast<float*>(out) + (int64_t)m * ldo + n;
+                    *o = add_rn(*o, y[t][r]);
+                }
+            }
+        }
+    }
+}
+
 // RA: the reassociated order (one activation scale per token, factored out of the block sum): per block
 // y = fma(float(P), sw, y), then y = RN(y sa) once; 2 VALU operations per output and block instead of 4.
-// PAN: `a` is the panel copy of q8_act_panel_kernel, so a wave's activation load for a stage is one 1 KB piece
-// (8 rows x 128 bytes of the tile's 16 KB stage chunk) instead of 8 rows' 128 bytes K apart.
-template <int EPI, bool RA, bool PAN = false>
-__global__ __launch_bounds__(256, 2) void w8a8_packed_tile_kernel(const int8_t* __restrict__ a,
+// PAN: `a` is the panel copy of q8_act_panel_kernel.
+template <int EPI, bool PAN = false>
+__global__ __launch_bounds__(256, 2) void w8a8_packed_reassoc_kernel(const int8_t* __restrict__ a,
                                                                   const float* __restrict__ a_s, int64_t as_sm,
                                                                   const int8_t* __restrict__ qt,
                                                                   const uint16_t* __restrict__ dt,
@@ -277,8 +484,8 @@ __global__ __launch_bounds__(256, 2) void w8a8_packed_tile_kernel(const int8_t* 
     const int8_t* ap[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        if (PAN) {                                   // the tile's panel: row lr + 32 i of each 16 KB stage chunk
-            ap[i] = a + (int64_t)m0 * K + (lr + 32 * i) * 128 + lc;
+        if (PAN) {                                   // the panel of row group m0 / 32 + i: row lr, the stage's bytes lc ..
+            ap[i] = a + (int64_t)(m0 + 32 * i) * K + (lc >> 5) * 1024 + ((lc >> 4) & 1) * 512 + lr * 16;
         } else {
             ap[i] = a + (int64_t)min(m0 + lr + 32 * i, M - 1) * K + lc;
         }
@@ -300,7 +507,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_packed_tile_kernel(const int8_t* 
     auto gload = [&](int kb) {                       // kb: first block of the stage (a multiple of 4)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            ra[i] = *reinterpret_cast<const v4i*>(ap[i] + (PAN ? (int64_t)(kb / 4) * 16384 : (int64_t)kb * 32));
+            ra[i] = *reinterpret_cast<const v4i*>(ap[i] + (PAN ? (int64_t)kb * 1024 : (int64_t)kb * 32));
             rb[i] = __builtin_nontemporal_load(bp[i] + (int64_t)(kb / 2) * 64);
         }
         rs = sp[(int64_t)(kb / 2) * 4];
@@ -317,7 +524,6 @@ __global__ __launch_bounds__(256, 2) void w8a8_packed_tile_kernel(const int8_t* 
                 sa[mt][r] = a_s[(int64_t)m * as_sm];
             }
     };
-    if (!RA) load_sa();                              // RA applies the scales once, after the K loop
     float y[2][2][16];
 #pragma unroll
     for (int mt = 0; mt < 2; mt++)
@@ -376,15 +582,12 @@ __global__ __launch_bounds__(256, 2) void w8a8_packed_tile_kernel(const int8_t* 
                     const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[mt], fb[nt], zero, 0, 0, 0);
 #pragma unroll
                     for (int r = 0; r < 16; r++) {
-                        if (RA)
-                            y[mt][nt][r] = __builtin_fmaf((float)acc[r], sw[nt], y[mt][nt][r]);
-                        else
-                            y[mt][nt][r] = add_rn(y[mt][nt][r], mul_rn(mul_rn((float)acc[r], sa[mt][r]), sw[nt]));
+                        y[mt][nt][r] = __builtin_fmaf((float)acc[r], sw[nt], y[mt][nt][r]);
                     }
                 }
         }
     }
-    if (RA) load_sa();
+    load_sa();                                       // the scales, applied once after the K loop
 #pragma unroll
     for (int mt = 0; mt < 2; mt++)
 #pragma unroll
@@ -395,7 +598,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_packed_tile_kernel(const int8_t* 
             for (int r = 0; r < 16; r++) {
                 const int m = m0 + wm * 64 + mt * 32 + 8 * (r >> 2) + lrow + (r & 3);
                 if (m < live) {
-                    if (RA) y[mt][nt][r] = mul_rn(y[mt][nt][r], sa[mt][r]);
+                    y[mt][nt][r] = mul_rn(y[mt][nt][r], sa[mt][r]);
                     if (EPI == 0) {
                         reinterpret_cast<uint16_t*>(out)[(int64_t)m * ldo + n] = (uint16_t)f32_to_bf16(y[mt][nt][r]);
                     } else {
@@ -552,23 +755,47 @@ static size_t packed_decode_lds(int R, int M) {
     return 2 * (size_t)R * M * 16 * 4 + 2 * (size_t)R * 16 * 4 + 2 * (size_t)M * (R * 32 + 16);
 }
 
-// Panel copy of the activations for w8a8_packed_tile_kernel<.., true>: 128-row tiles of K / 128 chunks of 16 KB, tile
-// t starting at byte 128 t K, chunk st holding rows 128 t .. + 127 (clamped to M - 1), inputs 128 st .. + 127,
-// row-major inside the chunk, so a tile's stage is one 16 KB piece.  One workgroup per (16 rows, 1024 inputs); each
-// row's 1 KB is read in one piece.
+// Panel copy of the activations for the tile kernels: 32-row groups of K / 32 blocks of 1 KB, a block's 16-byte piece l
+// being row l % 32 of the group (rows past M: row M - 1), inputs 16 (l / 32) .. + 15, so a wave's MFMA fragment of a block
+// is one 1 KB piece.  Rows up to a multiple of 128.  One workgroup per (32 rows, 512 inputs); each row's 512 bytes are
+// read in one piece.
 __global__ __launch_bounds__(256) void q8_act_panel_kernel(const int8_t* __restrict__ a, int8_t* __restrict__ pan,
                                                            int M, int K) {
     const int rb = blockIdx.y;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const int piece = threadIdx.x + 256 * j, r = piece >> 6;
-        const int k = 1024 * blockIdx.x + 16 * (piece & 63);
+        const int piece = threadIdx.x + 256 * j, r = piece >> 5;
+        const int k = 512 * blockIdx.x + 16 * (piece & 31);
         if (k >= K) continue;
-        const v4i v = *reinterpret_cast<const v4i*>(a + (int64_t)min(16 * rb + r, M - 1) * K + k);
-        const int row = 16 * rb + r;
-        *reinterpret_cast<v4i*>(pan + (int64_t)(row >> 7) * 128 * K + (int64_t)(k >> 7) * 16384 + (row & 127) * 128 +
-                                (k & 127)) = v;
+        const v4i v = *reinterpret_cast<const v4i*>(a + (int64_t)min(32 * rb + r, M - 1) * K + k);
+        *reinterpret_cast<v4i*>(pan + (int64_t)rb * 32 * K + (int64_t)(k >> 5) * 1024 + ((k >> 4) & 1) * 512 + r * 16) = v;
     }
+}
+
+// The exact tile kernel's column subtiles per wave (128 x 32 nt outputs per workgroup): the least time of the rounds of
+// 512 workgroups (two per CU).  Measured at K = 5120, a full round takes 115 / 87 / 64 us at 4 / 3 / 2 subtiles, and one
+// of at most a workgroup per CU 0.69 of that; wider tiles where they are within 5% (their last round overlaps the one
+// before it).  777 x 13824: 179 / 177 / 214 us; 300 x 13824: 101 / 87 / 103; 128 x 5120: 79 / 61 / 43; 8192 x 27648: 2996
+// / 3080 / 3518.  cost: the estimate in 10 ns at K = 5120.
+static int q8_tile_nt(int64_t M, int64_t N, int64_t* cost) {
+    const int64_t w[5] = {0, 0, 64, 87, 115};
+    int best = 4;
+    for (int nt = 4; nt >= 2; nt--) {
+        const int64_t t = (M + PBM - 1) / PBM * ((N + 32 * nt - 1) / (32 * nt)), rem = t % 512;
+        const int64_t c = w[nt] * (t / 512 * 100 + (rem == 0 ? 0 : rem <= 256 ? 69 : 100));
+        if (nt == 4 || c * 100 < *cost * 95) best = nt, *cost = c;
+    }
+    return best;
+}
+
+// Whether the register-fold kernel beats the tile kernel beyond 64 rows: it takes 16 x 32 outputs per wave and 21.7 ns a
+// wave at K = 5120 once they fill the chip (128 x 5120: 25 against 43 us; 128 x 13824: 75 against 80; 128 x 27648: 148
+// against 79; 300 x 1024: 17 against 43).
+static bool q8_mid_faster(int64_t M, int64_t N) {
+    int64_t tile = 0;
+    q8_tile_nt(M, N, &tile);
+    const int64_t mid = (M + 15) / 16 * ((N + 31) / 32) * 217 / 100;
+    return M <= 65535 * 16 && (mid < 1700 ? 1700 : mid) < tile;
 }
 
 // pan: the panel buffer for the tile kernels (kernels 0 and 3), or null for row-major activations
@@ -613,22 +840,28 @@ static void launch_packed(int kernel, const int8_t* a, const float* a_s, int64_t
             hipLaunchKernelGGL((w8a8_packed_mid_kernel<8, 1, 1, EPI>), dim3(N / 16, (M + 15) / 16), dim3(64), 0, st,
                                a, a_s, as_sm, qt, dt, out, ldo, n_rows, M, N, K);
     } else if (kernel == 0 || kernel == 3) {
-        const int tiles_m = (M + PBM - 1) / PBM, tiles_n = (N + PBN - 1) / PBN;
-        if (pan) {                                   // the panel copy first, then the tile kernel reads it
-            hipLaunchKernelGGL(q8_act_panel_kernel, dim3((unsigned)((K + 1023) / 1024), (unsigned)((M + 127) / 128 * 8)),
+        if (pan)                                     // the panel copy first, then the tile kernel reads it
+            hipLaunchKernelGGL(q8_act_panel_kernel, dim3((unsigned)((K + 511) / 512), (unsigned)((M + 127) / 128 * 4)),
                                dim3(256), 0, st, a, pan, M, K);
-            if (kernel == 0)
-                hipLaunchKernelGGL((w8a8_packed_tile_kernel<EPI, false, true>), dim3(tiles_m * tiles_n), dim3(256), 0,
-                                   st, pan, a_s, as_sm, qt, dt, out, ldo, n_rows, M, N, K, tiles_m, tiles_n);
-            else
-                hipLaunchKernelGGL((w8a8_packed_tile_kernel<EPI, true, true>), dim3(tiles_m * tiles_n), dim3(256), 0,
-                                   st, pan, a_s, as_sm, qt, dt, out, ldo, n_rows, M, N, K, tiles_m, tiles_n);
-        } else if (kernel == 0)
-            hipLaunchKernelGGL((w8a8_packed_tile_kernel<EPI, false>), dim3(tiles_m * tiles_n), dim3(256), 0, st, a,
-                               a_s, as_sm, qt, dt, out, ldo, n_rows, M, N, K, tiles_m, tiles_n);
-        else
-            hipLaunchKernelGGL((w8a8_packed_tile_kernel<EPI, true>), dim3(tiles_m * tiles_n), dim3(256), 0, st, a,
-                               a_s, as_sm, qt, dt, out, ldo, n_rows, M, N, K, tiles_m, tiles_n);
+        const int8_t* src = pan ? pan : a;
+        const int tiles_m = (M + PBM - 1) / PBM;
+#define Q8T(KER, BN)                                                                                               \
+    do {                                                                                                           \
+        const int tiles_n = (N + BN - 1) / BN;                                                                     \
+        hipLaunchKernelGGL((KER), dim3(tiles_m * tiles_n), dim3(256), 0, st, src, a_s, as_sm, qt, dt, out, ldo,    \
+                           n_rows, M, N, K, tiles_m, tiles_n);                                                     \
+    } while (0)
+        if (kernel == 3) {
+            if (pan) Q8T((w8a8_packed_reassoc_kernel<EPI, true>), PBN);
+            else Q8T((w8a8_packed_reassoc_kernel<EPI, false>), PBN);
+        } else {
+            int64_t cost = 0;
+            const int nt = q8_tile_nt(M, N, &cost);
+            if (nt == 4) { if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 4>), 128); else Q8T((w8a8_q8_tile_kernel<EPI, false, 4>), 128); }
+            else if (nt == 3) { if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 3>), 96); else Q8T((w8a8_q8_tile_kernel<EPI, false, 3>), 96); }
+            else { if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 2>), 64); else Q8T((w8a8_q8_tile_kernel<EPI, false, 2>), 64); }
+        }
+#undef Q8T
     }
 }
 
@@ -678,8 +911,9 @@ static int packed_gemm(const int8_t* a, const float* a_s, int64_t as_sm, const i
                             M * K < ((int64_t)1 << 31) && workspace &&
                             workspace_bytes >= q8_stream_workspace_bytes(N, K);
     // by default: the balanced kernel up to 16 rows (given its workspace), the row-round decode kernel up to 64 rows
-    // (and up to 16 without a workspace), the tile kernel beyond
-    if (kernel == -1) kernel = M >= 1 && M <= 16 && can_stream ? 4 : M <= 64 ? 1 : 0;
+    // (and up to 16 without a workspace), beyond them the register-fold kernel or the tile kernel
+    if (kernel == -1) kernel = M >= 1 && M <= 16 && can_stream ? 4 : M <= 64 ? 1 : q8_mid_faster(M, N) ? 2 : 0;
+    if (kernel == 0 && K > (1 << 23)) kernel = 2;      // the tile kernel's offsets within a tile are 32-bit; same bits
     if (kernel == 1 && M > 64) return PRISM_ERR_ARG;
     if (kernel == 4 && !can_stream) return M > 16 ? PRISM_ERR_SHAPE : PRISM_ERR_ARG;
     if (kernel == 2 && M > 65535 * 16) return PRISM_ERR_SHAPE;         // grid rows: one per 16 activation rows
