@@ -21,6 +21,7 @@
 #include "common.h"
 #include "w4a8_bal.h"
 #include "w4a8_common.h"
+#include "w4a8_mid.h"
 #include "w4a8_prefill.h"
 
 #ifndef Q4S_TG2_ROWS
@@ -871,8 +872,10 @@ extern "C" int prism_w4a8_q4k_gemm(const int8_t* xq, const float* a, int64_t a_s
     // a tile per workgroup leaves CUs with one tile more than others: 5120 x 17408 at 1 row 15.1 us against 18.4 us),
     // given its workspace; the per-tile kernel otherwise (13824 x 5120: 11.4 against 15.4 us; 5120^2 at 1-4 rows
     // 7.5-8.0 against 8.2-8.8 us) and from 5 rows, where it takes two tiles per workgroup (5120^2 at 16 rows 8.9
-    // against 9.9 us); the tile kernel beyond 16 rows.  The MI355X table overrides this per shape.
-    if (kernel == -1) kernel = M >= 1 && M <= 16 ? (can_bal && N / 16 < 512 && K >= 8192 && M <= 4 ? 2 : 1) : 0;
+    // against 9.9 us); beyond 16 rows the mid kernel (3, w4a8_mid.hip) where it is the faster one, else the tile kernel.  The
+    // MI355X table overrides this per shape up to 16 rows.
+    if (kernel == -1) kernel = M >= 1 && M <= 16 ? (can_bal && N / 16 < 512 && K >= 8192 && M <= 4 ? 2 : 1) :
+                                 w4_mid_faster(false, M, N, K) ? 3 : 0;
     if (kernel == 1 && M > 16) return PRISM_ERR_ARG;
     if (kernel == 2 && !can_bal) return M > 16 || !q4k_bal_fits(M, N, K) ? PRISM_ERR_SHAPE : PRISM_ERR_ARG;
     if (M == 0) return PRISM_OK;
@@ -908,6 +911,8 @@ extern "C" int prism_w4a8_q4k_gemm(const int8_t* xq, const float* a, int64_t a_s
         else { if (epi == 0) W4S_TG(4, 0); else W4S_TG(4, 1); }
 #undef W4S_TG
 #undef W4S
+    } else if (kernel == 3) {
+        w4_mid_launch(xq, a, a_sb, xs, qv, meta, out, ldo, n_rows, Mi, Ni, Ki, epi, st);
     } else if ((int64_t)(N / 16) * (K / 256) * 2048 < ((int64_t)1 << 31) && M * K < ((int64_t)1 << 31)) {
         // the 128 x 128 tile kernel (w4a8_prefill.hip), whose stage offsets are 32-bit
         q4k_tile_launch(xq, a, a_sb, xs, qv, meta, out, ldo, n_rows, Mi, Ni, Ki, epi, st);
@@ -945,8 +950,8 @@ extern "C" int prism_w4a8_q6k_gemm(const int8_t* xq, const float* a, int64_t a_s
         return PRISM_ERR_SHAPE;
     if (!PRISM_ALIGNED(xq, 16) || !PRISM_ALIGNED(qv, 16) || !PRISM_ALIGNED(meta, 16)) return PRISM_ERR_ALIGN;
     if (kernel < -1 || kernel > 2) return PRISM_ERR_ARG;
-    if (kernel == -1) kernel = M <= 16 ? 1 : 0;
-    if (kernel >= 1 && M > 16) return PRISM_ERR_ARG;
+    if (kernel == -1) kernel = M <= 16 ? 1 : w4_mid_faster(true, M, N, K) ? 3 : 0;
+    if ((kernel == 1 || kernel == 2) && M > 16) return PRISM_ERR_ARG;
     if (M == 0) return PRISM_OK;
     hipStream_t st = (hipStream_t)stream;
     const int Mi = (int)M, Ni = (int)N, Ki = (int)K;
@@ -991,6 +996,8 @@ extern "C" int prism_w4a8_q6k_gemm(const int8_t* xq, const float* a, int64_t a_s
         }
 #undef Q6DEC_
 #undef Q6DEC
+    } else if (kernel == 3) {
+        w4_mid_launch(xq, a, a_sb, nullptr, qv, meta, out, ldo, n_rows, Mi, Ni, Ki, epi, st);
     } else if ((int64_t)(N / 16) * (K / 256) * 4096 < ((int64_t)1 << 31) && M * K < ((int64_t)1 << 31)) {
         // the 128 x 128 two-plane tile kernel (w4a8_prefill.hip), whose stage offsets are 32-bit
         q6k_tile_launch(xq, a, a_sb, qv, meta, out, ldo, n_rows, Mi, Ni, Ki, epi, st);

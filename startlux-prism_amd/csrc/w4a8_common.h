@@ -41,6 +41,21 @@ constexpr int Q6_META = 288;
 
 __device__ __forceinline__ int sbyte(v4u m, int j) { return (int)(int8_t)(m[j >> 2] >> (8 * (j & 3))); }
 
+// Four signed weights (bytes of v) times the scale pair sc16 (sc in both 16-bit halves) as the two plane dwords
+// (w & 63, w >> 6) in byte order.
+__device__ __forceinline__ void q6_planes(uint32_t v, uint32_t sc16, uint32_t& lo, uint32_t& hi) {
+    typedef short s2 __attribute__((ext_vector_type(2)));
+    const s2 ev = __builtin_bit_cast(s2, v << 8) >> (s2){8, 8};       // bytes 0, 2 sign-extended
+    const s2 od = __builtin_bit_cast(s2, v) >> (s2){8, 8};            // bytes 1, 3
+    const s2 sc = __builtin_bit_cast(s2, sc16);
+    const s2 we = ev * sc, wo = od * sc;                              // |w| <= 4096: exact in 16 bits
+    const uint32_t le = __builtin_bit_cast(uint32_t, we) & 0x003f003fu, lo_ = __builtin_bit_cast(uint32_t, wo) & 0x003f003fu;
+    const uint32_t he = __builtin_bit_cast(uint32_t, (s2)(we >> (s2){6, 6}));
+    const uint32_t ho = __builtin_bit_cast(uint32_t, (s2)(wo >> (s2){6, 6}));
+    lo = __builtin_amdgcn_perm(lo_, le, 0x06020400u);                  // bytes e0 o0 e1 o1
+    hi = __builtin_amdgcn_perm(ho, he, 0x06020400u);
+}
+
 // One row's 16 meta bytes -> d, dmin (fp32) and the 8 scales and 8 mins (ggml get_scale_min_k4).
 __device__ __forceinline__ void row_meta(v4u m, float& d, float& dm, int* sc, int* mn) {
     d = f16_to_f32(m[0] & 0xffffu);

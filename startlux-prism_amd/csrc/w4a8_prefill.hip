@@ -284,21 +284,6 @@ __global__ __launch_bounds__(512, 1) void w4a8_q4k_tile_kernel(const int8_t* __r
 // A lane's operand for inputs 64 p + 16 q .. + 15 is two 8-byte pieces of the packed chunk p: lane slots
 // 32 (q & 1) + lm and 32 (q & 1) + 16 + lm, bytes 8 (q >> 1) .. + 7 of each.
 
-// Four signed weights (bytes of v) times the scale pair sc16 (sc in both 16-bit halves) as the two plane dwords
-// (w & 63, w >> 6) in byte order.
-__device__ __forceinline__ void q6_planes(uint32_t v, uint32_t sc16, uint32_t& lo, uint32_t& hi) {
-    typedef short s2 __attribute__((ext_vector_type(2)));
-    const s2 ev = __builtin_bit_cast(s2, v << 8) >> (s2){8, 8};       // bytes 0, 2 sign-extended
-    const s2 od = __builtin_bit_cast(s2, v) >> (s2){8, 8};            // bytes 1, 3
-    const s2 sc = __builtin_bit_cast(s2, sc16);
-    const s2 we = ev * sc, wo = od * sc;                              // |w| <= 4096: exact in 16 bits
-    const uint32_t le = __builtin_bit_cast(uint32_t, we) & 0x003f003fu, lo_ = __builtin_bit_cast(uint32_t, wo) & 0x003f003fu;
-    const uint32_t he = __builtin_bit_cast(uint32_t, (s2)(we >> (s2){6, 6}));
-    const uint32_t ho = __builtin_bit_cast(uint32_t, (s2)(wo >> (s2){6, 6}));
-    lo = __builtin_amdgcn_perm(lo_, le, 0x06020400u);                  // bytes e0 o0 e1 o1
-    hi = __builtin_amdgcn_perm(ho, he, 0x06020400u);
-}
-
 template <int EPI>
 __global__ __launch_bounds__(512, 1) void w4a8_q6k_tile_kernel(const int8_t* __restrict__ xq,
                                                                 const float* __restrict__ a, int64_t a_sb,
