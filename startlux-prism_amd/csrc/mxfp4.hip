@@ -890,6 +890,211 @@ int64_t mx_split_workspace_bytes(int64_t N, int64_t K) {     // 1 KB of segment 
     return nseg > 1 ? nseg * T * 1024 : 16;
 }
 
+// ------------------------------------------------------------------------------ mid kernel
+// Batches of 17 rows and more on projections whose 64 x 256 tiles do not fill the chip, and e2m1 batches up to 16 rows.
+// A workgroup owns TG adjacent 16-row weight tiles and MT 16-row activation tiles; its waves take the 1024-input segments
+// in turn (wave w segment r NW + w of round r), each for all TG x MT blocks, and leave the segment sums in LDS, where
+// after one barrier per round wave b adds block b's sums left to right.  The decode kernel it replaces here had one tile
+// per workgroup, so every weight byte cost MT activation bytes (e2m1), loaded a row per lane: the memory pipeline merges
+// neighbouring lanes only, so each piece was an access of its own.  Here four neighbouring lanes load a row's 64 bytes
+// and the wave turns them in LDS (piece c of row r at slot c ^ mx_turn(r / 4): the read's lane groups, 0-3, 12-15, 20-27
+// and the others of 32, then lie on distinct banks), and the TG tiles share them.  Both operands are requested four steps
+// ahead.  Same MFMA chain per segment and segment order: the same bits.
+__device__ __forceinline__ int mx_turn(int r4) { return ((r4 ^ (r4 << 1)) & 2) | (r4 >> 1); }
+constexpr int kMxMidWaves = 8;
+
+template <int AF, int TG, int MT, int EPI>
+__global__ __launch_bounds__(64 * kMxMidWaves, 2) void mx_mid_kernel(const uint8_t* __restrict__ aq,
+                                                                    const uint8_t* __restrict__ as,
+                                                                    const uint8_t* __restrict__ wq,
+                                                                    const uint8_t* __restrict__ ws,
+                                                                    void* __restrict__ out, int64_t ldo,
+                                                                    const int32_t* __restrict__ n_rows, int M, int N,
+                                                                    int K, int gy) {
+    constexpr int AP = AF == 0 ? 2 : 1, NB = TG * MT;      // 64-byte halves of an activation row's step; blocks
+    extern __shared__ __attribute__((aligned(16))) uint8_t dsm[];
+    const int NW = blockDim.x >> 6, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    v4f* sums = reinterpret_cast<v4f*>(dsm);               // [2][NW][NB][64]
+    uint8_t* xw = dsm + (size_t)2 * NW * NB * 1024 + wv * MT * 1024;
+    const int p = lane >> 4, r = lane & 15;
+    // the row groups of one tile group run on one XCD next to each other, so its weights come from HBM once
+    const int j8 = blockIdx.x >> 3, nt0 = ((j8 / gy) * 8 + (blockIdx.x & 7)) * TG, m0 = (j8 % gy) * 16 * MT;
+    if (nt0 * 16 >= N) return;
+    if (m0 > 0 && n_rows && m0 >= __ldg(n_rows)) return;
+    const int KS = K / kMxStep, nseg = (KS + kMxSegSteps - 1) / kMxSegSteps, nr = (nseg + NW - 1) / NW;
+    const int abytes = AF == 0 ? K : K / 2;
+
+    const auto rw = buf_rsrc(wq + (int64_t)nt0 * KS * 1024), rws = buf_rsrc(ws + (int64_t)nt0 * KS * 64);
+    const auto ra = buf_rsrc(aq + (int64_t)m0 * abytes);
+    // (bounded: the last group of four steps' scales may reach past the last row when K / 128 is not a multiple of 4)
+    const auto rs = buf_rsrc_n(as + (int64_t)m0 * (K / 32), (uint32_t)min((int64_t)(M - m0) * (K / 32), (int64_t)0x7fffffff));
+    uint32_t av[MT], sv[MT];
+#pragma unroll
+    for (int j = 0; j < MT; j++) {
+        av[j] = (uint32_t)(min(m0 + 16 * j + (lane >> 2), M - 1) - m0) * abytes + 16 * ((lane & 3) ^ mx_turn(lane >> 4));
+        sv[j] = (uint32_t)(min(m0 + 16 * j + r, M - 1) - m0) * (K / 32);
+    }
+    const int xrd = r * 64 + 16 * (p ^ mx_turn(r >> 2));
+
+    v4i w[4][TG], x[4][MT][AP];
+    uint32_t wsc[4][TG];
+    v4u xs[2][MT];
+    // step j of segment s, clamped to the last step (redundant requests past the end)
+    auto load_w = [&](int s, int j) {
+        const int st = min(s * kMxSegSteps + j, KS - 1);
+#pragma unroll
+        for (int g = 0; g < TG; g++) {
+            w[j & 3][g] = buf_load16<kBufNT>(rw, lane * 16, (g * KS + st) * 1024);
+            wsc[j & 3][g] = buf_load1(rws, lane, (g * KS + st) * 64);
+        }
+    };
+    auto load_x = [&](int s, int j) {
+        const int st = min(s * kMxSegSteps + j, KS - 1);
+        if ((j & 3) == 0) {
+#pragma unroll
+            for (int c = 0; c < MT; c++) xs[(j >> 2) & 1][c] = __builtin_bit_cast(v4u, buf_load16(rs, sv[c], (st & ~3) * 4));
+        }
+#pragma unroll
+        for (int c = 0; c < MT; c++)
+#pragma unroll
+            for (int h = 0; h < AP; h++) x[j & 3][c][h] = buf_load16(ra, av[c], st * 64 * AP + 64 * h);
+    };
+    v4f y[NB];                                             // wave b < NB: block b, b + NW, ...
+    auto fold = [&](int rd) {
+        const int n = min(NW, nseg - rd * NW);
+        const v4f* sb = sums + (size_t)(rd & 1) * NW * NB * 64 + lane;
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            const int b = wv + k * NW;
+            if (b < NB) {
+                for (int i = 0; i < n; i++) {
+                    const v4f z = sb[((size_t)i * NB + b) * 64];
+                    y[k] = rd == 0 && i == 0 ? z : v4f{add_rn(y[k].x, z.x), add_rn(y[k].y, z.y), add_rn(y[k].z, z.z),
+                                                       add_rn(y[k].w, z.w)};
+                }
+            }
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < 4; j++) load_w(wv, j);
+#pragma unroll
+    for (int j = 0; j < 4; j++) load_x(wv, j);
+    for (int rd = 0; rd < nr; rd++) {
+        const int s = rd * NW + wv, left = KS - s * kMxSegSteps;         // this wave's steps (none past the last segment)
+        v4f acc[TG][MT];
+#pragma unroll
+        for (int g = 0; g < TG; g++)
+#pragma unroll
+            for (int c = 0; c < MT; c++) acc[g][c] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            // this step's pieces to LDS and back as MFMA operands (the wave's LDS operations run in order)
+            v4i xo[MT][AP];
+#pragma unroll
+            for (int h = 0; h < AP; h++) {
+#pragma unroll
+                for (int c = 0; c < MT; c++) *reinterpret_cast<v4i*>(xw + c * 1024 + lane * 16) = x[j & 3][c][h];
+#pragma unroll
+                for (int c = 0; c < MT; c++) xo[c][h] = *reinterpret_cast<const v4i*>(xw + c * 1024 + xrd);
+            }
+            uint32_t sc[MT];
+#pragma unroll
+            for (int c = 0; c < MT; c++) sc[c] = __builtin_amdgcn_ubfe(xs[(j >> 2) & 1][c][j & 3], 8 * p, 8);
+            const bool more = j < 4 || rd + 1 < nr;
+            if (more) load_x(j < 4 ? s : s + NW, (j + 4) & 7);
+            if (j < left) {
+#pragma unroll
+                for (int c = 0; c < MT; c++) {
+                    v8i a = {xo[c][0].x, xo[c][0].y, xo[c][0].z, xo[c][0].w, 0, 0, 0, 0};
+                    if constexpr (AF == 0) a[4] = xo[c][1].x, a[5] = xo[c][1].y, a[6] = xo[c][1].z, a[7] = xo[c][1].w;
+#pragma unroll
+                    for (int g = 0; g < TG; g++) acc[g][c] = mx_mfma<AF>(w[j & 3][g], a, acc[g][c], wsc[j & 3][g], sc[c]);
+                }
+            }
+            if (more) load_w(j < 4 ? s : s + NW, (j + 4) & 7);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        v4f* sb = sums + ((size_t)((rd & 1) * NW + wv) * NB) * 64 + lane;
+#pragma unroll
+        for (int g = 0; g < TG; g++)
+#pragma unroll
+            for (int c = 0; c < MT; c++) sb[(g * MT + c) * 64] = acc[g][c];
+        lds_barrier();
+        fold(rd);
+    }
+    const int live = n_rows ? min(M, __ldg(n_rows)) : M;
+#pragma unroll
+    for (int k = 0; k < NB; k++) {
+        const int b = wv + k * NW;
+        if (b < NB) {
+            const int m = m0 + 16 * (b % MT) + r;
+            if (m < live) mx_store<EPI>(out, ldo, m, 16 * (nt0 + b / MT) + 4 * p, y[k]);
+        }
+    }
+}
+
+template <int AF, int TG, int MT, int EPI>
+static void mx_mid_go(int nw, const uint8_t* aq, const uint8_t* as, const uint8_t* wq, const uint8_t* ws, void* out,
+                      int64_t ldo, const int32_t* n_rows, int M, int N, int K, int gy, hipStream_t st) {
+    const size_t lds = (size_t)nw * (2 * TG * MT + MT) * 1024;
+    allow_lds(mx_mid_kernel<AF, TG, MT, EPI>, lds);
+    hipLaunchKernelGGL((mx_mid_kernel<AF, TG, MT, EPI>), dim3((unsigned)((N / 16 / TG + 7) / 8 * 8 * gy)), dim3(64 * nw),
+                       lds, st, aq, as, wq, ws, out, ldo, n_rows, M, N, K, gy);
+}
+
+// 16-row activation tiles per workgroup: up to four of e2m1 rows, three of e4m3 (four spill registers: 64 x 13824 x 5120
+// 47 us), in equal row groups.
+struct MxMidRows {
+    int gy, mt;
+    MxMidRows(int a_fmt, int64_t M) {
+        const int64_t t = (M + 15) / 16, most = a_fmt == PRISM_MX_E2M1 ? 4 : 3;
+        gy = (int)((t + most - 1) / most);
+        mt = (int)((t + gy - 1) / gy);
+    }
+};
+
+// Two weight tiles per workgroup share each activation piece (24 x 34816 x 5120 e2m1 28 us against 34 with one, 24 x
+// 5120 x 17408 19 against 24; four tiles 28 and 26); one where N / 16 is odd.
+template <int AF>
+static void mx_mid_launch(const uint8_t* aq, const uint8_t* as, const uint8_t* wq, const uint8_t* ws, void* out,
+                          int64_t ldo, const int32_t* n_rows, int M, int N, int K, int epi, hipStream_t st) {
+    const MxMidRows rows(AF, M);
+    const int gy = rows.gy, mt = rows.mt;
+    const int nseg = (K / kMxStep + kMxSegSteps - 1) / kMxSegSteps, rounds = (nseg + kMxMidWaves - 1) / kMxMidWaves;
+    const int nw = (nseg + rounds - 1) / rounds;           // equal rounds
+    constexpr int M4 = AF == 0 ? 3 : 4;
+#define MXM(TGV, MTV)                                                                                                \
+    do {                                                                                                             \
+        if (epi) mx_mid_go<AF, TGV, MTV, 1>(nw, aq, as, wq, ws, out, ldo, n_rows, M, N, K, gy, st);                  \
+        else mx_mid_go<AF, TGV, MTV, 0>(nw, aq, as, wq, ws, out, ldo, n_rows, M, N, K, gy, st);                      \
+    } while (0)
+#define MXM_MT(TGV)                                                                                                  \
+    do {                                                                                                             \
+        if (mt == 1) MXM(TGV, 1); else if (mt == 2) MXM(TGV, 2); else if (mt == 3) MXM(TGV, 3); else MXM(TGV, M4);   \
+    } while (0)
+    if (N % 32 == 0) MXM_MT(2);
+    else MXM_MT(1);
+#undef MXM_MT
+#undef MXM
+}
+
+// Whether the mid kernel takes the shape.  Up to 16 rows: e2m1 batches from 20 M weights (16 x 34816 x 5120 30.1 -> 21.7 us,
+// 5120^2 at 1 / 16 rows 6.2 / 9.2 -> 5.6 / 6.8; 1 x 1024 x 5120 3.8 against 4.7), and of e4m3 the wide ones the split
+// decode would take (34816 x 5120 at 1 / 16 rows 26.3 / 25.9 -> 19.9 / 22.9 us; at 5120 x 17408 and 16 rows the split stays
+// ahead, 16.7 against 17.5).  Beyond, from 8 M weights (17 x 1024 x 2048 4.1 against 4.6), measured at K = 5120 (both sides go with K): about 3 us and
+// 5.6 ns (e2m1) or 7.2 ns (e4m3) per 16 x 16 outputs, against the tile kernel's 21 us and 75 ns per 64 x 256 tile up to
+// one per CU, 45 us per round of two beyond (us, mid / tile: e2m1 24 x 34816 28.1 / 27.9, 64 x 13824 21 / 29, 128 x 5120
+// 19.1 / 20.3, 128 x 13824 37 / 28; e4m3 32 x 13824 16 / 27.5, 40 x 5120 10.5 / 22).
+static bool mx_mid_faster(int a_fmt, int64_t M, int64_t N, int64_t K, bool split) {
+    if (a_fmt == PRISM_MX_E4M3_PANELS || K > (1 << 22) || M > (1 << 16)) return false;    // 32-bit offsets
+    if (M <= 16) return a_fmt == PRISM_MX_E2M1 ? N * K >= (20LL << 20) : split && N > 8192;
+    if (N * K < (8LL << 20)) return false;
+    const MxMidRows rows(a_fmt, M);
+    const int64_t blocks = (int64_t)rows.gy * rows.mt * (N / 16), tiles = (M + 63) / 64 * ((N + 255) / 256);
+    const int64_t mid = 3000 + blocks * (a_fmt == PRISM_MX_E2M1 ? 56 : 72) / 10;
+    return mid < (tiles <= 256 ? 21000 + 75 * tiles : (tiles + 511) / 512 * 45000);
+}
+
 static size_t mx_decode_lds(int MT, int K) {
     const int nseg = (K / kMxStep + kMxSegSteps - 1) / kMxSegSteps;
     return (size_t)nseg * MT * 64 * sizeof(v4f);
@@ -979,6 +1184,12 @@ extern "C" int prism_mxfp4_gemm_ws(const uint8_t* aq, const uint8_t* as, int a_f
     // measured against the staged decode at 1-16 rows: 15.8-16.0 against 17.3-18.8 us at 17408 x 5120, 16.9
     // against 18.2-20.6 at 5120 x 17408, 21.5-21.7 against 23.5-25.6 at 27648 x 5120; slower below about 80 M weights
     // (its second launch costs about 2.5 us: 8.5 against 6.7-7.3 us at 5120^2, 14.0 against 11.4 at 8192^2)
+    if (kernel < 0 && PRISM_ALIGNED(as, 4) && mx_mid_faster(a_fmt, M, N, K, split_ok && N * K >= (80LL << 20))) {
+        if (a_fmt == PRISM_MX_E4M3) mx_mid_launch<0>(aq, as, wq, ws, out, ldo, n_rows, (int)M, (int)N, (int)K, epi, st);
+        else mx_mid_launch<4>(aq, as, wq, ws, out, ldo, n_rows, (int)M, (int)N, (int)K, epi, st);
+        PRISM_LAUNCH_CHECK();
+        return PRISM_OK;
+    }
     if (kernel < 0 && split_ok && N * K >= (80LL << 20)) kernel = 2;
     if (kernel < 0) kernel = (MT <= 4 && mx_decode_lds(MT, (int)K) <= 64 * 1024) ? 1 : 0;
     if (kernel == 2) {
