@@ -55,16 +55,6 @@ __device__ __forceinline__ int ilog2_ceil(float v) {
     return (int)((u >> 23) & 0xff) - 127 + ((u & 0x7fffffu) != 0);
 }
 
-// fp32 (|v| <= 448) -> e4m3 code, round to nearest even; the sign bit follows the input's.
-__device__ __forceinline__ uint32_t e4m3_code(float v) {
-    const uint32_t sgn = (__float_as_uint(v) >> 24) & 0x80u;
-    const float a = fabsf(v);
-    if (a < 0x1p-6f) return sgn | (uint32_t)__builtin_rintf(a * 512.f);
-    const int E = ilog2_floor(a);
-    const uint32_t m = (uint32_t)__builtin_rintf(a * pow2i(3 - E));
-    return sgn | (uint32_t)((E + 6) * 8 + (int)m);
-}
-
 // ------------------------------------------------------------------------------------------------ weight pack
 // fp32 [N, K] (row stride ldw) -> device layout.  One workgroup of 64 threads per (16-row tile, 128-input step);
 // thread L quantizes row 16 t + L % 16, block 4 s + L / 16 and writes its 16 code bytes and scale byte.
@@ -149,85 +139,86 @@ __host__ __device__ __forceinline__ int64_t mx_act_panel_offset(int64_t row, int
     return (row >> 4) * 16 * K + st * 2048 + h * 1024 + (16 * p + (row & 15)) * 16 + (k & 15);
 }
 
-// One thread per (row, 32-input block).  AF 4: kernels/mxfp4.py:124-146 (_quant_kernel; with inv, :149-170
-// _quant_scaled_kernel): e = clip(ceil(log2(max(amax, 1e-30) / 6)), +-127), strict-threshold codes, the sign bit
-// set for every negative input.  AF 0: tests/quant_sim.py:75-81 (mxfp8): e = floor(log2(max(amax, 1e-30))) - 8,
+// Four neighbouring lanes per (row, 32-input block), 8 inputs each.  AF 4: kernels/mxfp4.py:124-146 (_quant_kernel; with
+// inv, :149-170 _quant_scaled_kernel): e = clip(ceil(log2(max(amax, 1e-30) / 6)), +-127), strict-threshold codes, the
+// sign bit set for every negative input.  AF 0: tests/quant_sim.py:75-81 (mxfp8): e = floor(log2(max(amax, 1e-30))) - 8,
 // codes e4m3(clamp(x / 2^e, +-448)) nearest even.  XF32: fp32 input, else bf16.  Rows >= n_rows are skipped.
 // PAN (e4m3 only): q in the panel layout mx_act_panel_offset defines instead of row-major.
+// Memory bounds it.  A thread per block read 64 bytes on its own, one 64-byte line per lane and load, and left a panel
+// chunk's stores to sixteen workgroups; here a wave's loads are contiguous (1 KB of bf16), and a panel workgroup owns
+// whole 2 KB chunks: 16 rows x 128 inputs, four of them requested at once.
 template <int AF, bool XF32, bool PAN = false>
 __global__ __launch_bounds__(256) void mx_quant_act_kernel(const void* __restrict__ x, int64_t ldx,
                                                            const float* __restrict__ inv, uint8_t* __restrict__ q,
                                                            uint8_t* __restrict__ s,
                                                            const int32_t* __restrict__ n_rows, int M, int K) {
-    const int row = blockIdx.y;
-    const int blk = blockIdx.x * blockDim.x + threadIdx.x;
-    const int live = n_rows ? min(M, __ldg(n_rows)) : M;
-    if (row >= live || blk >= K / 32) return;
-    float v[32];
-    if (XF32) {
-        const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(x) + row * ldx + 32 * blk);
+    constexpr int U = PAN ? 4 : 1;                         // 8-input pieces per thread
+    const int tid = threadIdx.x;
+    const int row = PAN ? blockIdx.y * 16 + (tid >> 4) : blockIdx.y;
+    int k[U];                                              // piece u: inputs k[u] .. + 7 (whole 32-input blocks in range)
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float4 f = src[i];
-            v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
-        }
-    } else {
-        const v4u* src = reinterpret_cast<const v4u*>(static_cast<const uint16_t*>(x) + row * ldx + 32 * blk);
+    for (int u = 0; u < U; u++) k[u] = PAN ? (blockIdx.x * U + u) * 128 + (tid & 15) * 8 : (blockIdx.x * 256 + tid) * 8;
+    float v[U][8];
+    const int64_t lrow = min(row, M - 1);                  // loads first, in range; the row count is read under them
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const v4u u = src[i];
+    for (int u = 0; u < U; u++) {
+        const int kk = min(k[u], K - 8);
+        if (XF32) {
+            const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(x) + lrow * ldx + kk);
+            const float4 a = src[0], b = src[1];
+            v[u][0] = a.x; v[u][1] = a.y; v[u][2] = a.z; v[u][3] = a.w;
+            v[u][4] = b.x; v[u][5] = b.y; v[u][6] = b.z; v[u][7] = b.w;
+        } else {
+            const v4u w = *reinterpret_cast<const v4u*>(static_cast<const uint16_t*>(x) + lrow * ldx + kk);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                v[8 * i + 2 * j] = bf16_to_f32(u[j] & 0xffffu);
-                v[8 * i + 2 * j + 1] = bf16_to_f32(u[j] >> 16);
+                v[u][2 * j] = bf16_to_f32(w[j] & 0xffffu);
+                v[u][2 * j + 1] = bf16_to_f32(w[j] >> 16);
             }
         }
-    }
-    if (inv) {
-        const float4* iv = reinterpret_cast<const float4*>(inv + 32 * blk);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float4 f = iv[i];
-            v[4 * i] = mul_rn(v[4 * i], f.x);
-            v[4 * i + 1] = mul_rn(v[4 * i + 1], f.y);
-            v[4 * i + 2] = mul_rn(v[4 * i + 2], f.z);
-            v[4 * i + 3] = mul_rn(v[4 * i + 3], f.w);
+        if (inv) {
+            const float4* iv = reinterpret_cast<const float4*>(inv + kk);
+            const float4 a = iv[0], b = iv[1];
+            v[u][0] = mul_rn(v[u][0], a.x); v[u][1] = mul_rn(v[u][1], a.y);
+            v[u][2] = mul_rn(v[u][2], a.z); v[u][3] = mul_rn(v[u][3], a.w);
+            v[u][4] = mul_rn(v[u][4], b.x); v[u][5] = mul_rn(v[u][5], b.y);
+            v[u][6] = mul_rn(v[u][6], b.z); v[u][7] = mul_rn(v[u][7], b.w);
         }
     }
-    float amax = 0.f;
+    const int live = n_rows ? min(M, __ldg(n_rows)) : M;
 #pragma unroll
-    for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(v[i]));
-    int e;
-    if (AF == 0) {
-        e = ilog2_floor(fmaxf(amax, 1e-30f)) - 8;
-        const float r = pow2i(-e);
-        uint32_t words[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int u = 0; u < U; u++) {
+        float amax = 0.f;
 #pragma unroll
-        for (int i = 0; i < 32; i++) {
-            const float a = fminf(fmaxf(v[i] * r, -448.f), 448.f);
-            words[i >> 2] |= e4m3_code(a) << (8 * (i & 3));
-        }
-        if (PAN) {                                         // the block's two 16-byte pieces p = 2 (blk % 2) + 0, 1
-            uint8_t* d = q + mx_act_panel_offset(row, 32 * blk, K);
-            *reinterpret_cast<v4u*>(d) = v4u{words[0], words[1], words[2], words[3]};
-            *reinterpret_cast<v4u*>(d + 256) = v4u{words[4], words[5], words[6], words[7]};
+        for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[u][i]));
+        amax = fmaxf(amax, __shfl_xor(amax, 1, kWave));    // the block's four lanes
+        amax = fmaxf(amax, __shfl_xor(amax, 2, kWave));
+        if (row >= live || k[u] >= K) continue;
+        int e;
+        if (AF == 0) {
+            e = ilog2_floor(fmaxf(amax, 1e-30f)) - 8;
+            const float r = pow2i(-e);
+            float c[8];                                    // v_cvt_pk_fp8_f32: e4m3, nearest even, subnormals and -0 kept
+#pragma unroll
+            for (int i = 0; i < 8; i++) c[i] = fminf(fmaxf(v[u][i] * r, -448.f), 448.f);
+            uint32_t w[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(c[4 * h], c[4 * h + 1], 0, false);
+                w[h] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c[4 * h + 2], c[4 * h + 3], lo, true);
+            }
+            uint8_t* d = PAN ? q + mx_act_panel_offset(row, k[u], K) : q + (int64_t)row * K + k[u];
+            *reinterpret_cast<v2u*>(d) = v2u{w[0], w[1]};
         } else {
-            v4u* dst = reinterpret_cast<v4u*>(q + (int64_t)row * K + 32 * blk);
-            dst[0] = v4u{words[0], words[1], words[2], words[3]};
-            dst[1] = v4u{words[4], words[5], words[6], words[7]};
-        }
-    } else {
-        e = min(127, max(-127, ilog2_ceil(div_rn(fmaxf(amax, 1e-30f), 6.0f))));
-        const float r = pow2i(-e);
-        uint32_t words[4] = {0, 0, 0, 0};
+            e = min(127, max(-127, ilog2_ceil(div_rn(fmaxf(amax, 1e-30f), 6.0f))));
+            const float r = pow2i(-e);
+            uint32_t w = 0;
 #pragma unroll
-        for (int i = 0; i < 32; i++) {
-            const uint32_t c = e2m1_mag<0>(fabsf(v[i]) * r) | (v[i] < 0.f ? 8u : 0u);
-            words[i >> 3] |= c << (4 * (i & 7));
+            for (int i = 0; i < 8; i++) w |= (e2m1_mag<0>(fabsf(v[u][i]) * r) | (v[u][i] < 0.f ? 8u : 0u)) << (4 * i);
+            *reinterpret_cast<uint32_t*>(q + (int64_t)row * (K / 2) + k[u] / 2) = w;
         }
-        *reinterpret_cast<v4u*>(q + (int64_t)row * (K / 2) + 16 * blk) = v4u{words[0], words[1], words[2], words[3]};
+        if ((tid & 3) == 0) s[(int64_t)row * (K / 32) + k[u] / 32] = (uint8_t)(e + 127);
     }
-    s[(int64_t)row * (K / 32) + blk] = (uint8_t)(e + 127);
 }
 
 // ------------------------------------------------------------------------------------------------ MFMA helpers
@@ -1141,7 +1132,8 @@ extern "C" int prism_mxfp4_quant_act(const void* x, int x_f32, int64_t ldx, cons
         (inv && !PRISM_ALIGNED(inv, 16)))
         return PRISM_ERR_ALIGN;
     if (M == 0) return PRISM_OK;
-    dim3 grid((unsigned)((K / 32 + 255) / 256), (unsigned)M);
+    const dim3 grid = fmt == PRISM_MX_E4M3_PANELS ? dim3((unsigned)((K + 511) / 512), (unsigned)((M + 15) / 16))
+                                                  : dim3((unsigned)((K + 2047) / 2048), (unsigned)M);
     hipStream_t st = (hipStream_t)stream;
 #define QA(AF, F) hipLaunchKernelGGL((mx_quant_act_kernel<AF, F>), grid, dim3(256), 0, st, x, ldx, inv, q, s, n_rows, \
                                      (int)M, (int)K)
