@@ -546,19 +546,22 @@ extern "C" int prism_swiglu_quant(const void* gu, int gu_f32, int64_t ldg, const
     if (gu_f32 && FF % 4) return PRISM_ERR_SHAPE;
     if (M == 0) return PRISM_OK;
     hipStream_t st = (hipStream_t)stream;
-    // few rows (decode): 1024 threads per row; the results do not depend on the workgroup size
-    const bool wide = M <= 64;
+    // few rows (decode): 1024 threads per row; rows longer than 4096: 512 (the exp and the divisions bound the kernel, and
+    // at 256 threads a lane holds so many chunks that two waves fit a SIMD: 1500 x 17408 49 -> 37 us, 8192 x 13824 168 ->
+    // 142, 5000 x 8192 51 -> 47; 1024 threads 45 / 143 / 53; at 2000 x 4096 no difference).  The results do not depend on it.
+    const int tpb = M <= 64 ? 1024 : FF > 4096 ? 512 : kPThreads;
     return pick_nch((int)FF, [&](auto nc) {
         constexpr int NC = decltype(nc)::value;
 #define SW(B, G32, T) hipLaunchKernelGGL((swiglu_prod_kernel<NC, B, G32, T>), dim3((unsigned)M), dim3(T), 0, st, gu,  \
                                          ldg, inv_s, q, s, xs, n_rows, (int)M, (int)FF)
-#define SWT(B, G32) do { if (wide) SW(B, G32, 1024); else SW(B, G32, kPThreads); } while (0)
+#define SWT(B, G32) do { if (tpb == 1024) SW(B, G32, 1024); else if (tpb == 512) SW(B, G32, 512); \
+                         else SW(B, G32, kPThreads); } while (0)
         if (gu_f32) { if (back == 0) SWT(0, true); else if (back == 1) SWT(1, true); else SWT(2, true); }
         else { if (back == 0) SWT(0, false); else if (back == 1) SWT(1, false); else SWT(2, false); }
 #undef SWT
 #undef SW
         return hipGetLastError() == hipSuccess ? 0 : (int)PRISM_ERR_LAUNCH;
-    }, wide ? 1024 : kPThreads);
+    }, tpb);
 }
 
 // back as prism_norm_quant.  o: the GDN output rows, z: the gate values of the row (the projection row plus the
