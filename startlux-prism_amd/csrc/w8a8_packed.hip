@@ -788,9 +788,10 @@ static int q8_tile_nt(int64_t M, int64_t N, int64_t* cost) {
     return best;
 }
 
-// Whether the register-fold kernel beats the tile kernel beyond 64 rows: it takes 16 x 32 outputs per wave and 21.7 ns a
+// Whether the register-fold kernel beats the tile kernel beyond 16 rows: it takes 16 x 32 outputs per wave and 21.7 ns a
 // wave at K = 5120 once they fill the chip (128 x 5120: 25 against 43 us; 128 x 13824: 75 against 80; 128 x 27648: 148
-// against 79; 300 x 1024: 17 against 43).
+// against 79; 32 x 34816 76 against 62; 300 x 1024: 17 against 43).  Over the dispatch table's 320 shapes and row counts the
+// choice costs 0.3% on average against the faster of the two.
 static bool q8_mid_faster(int64_t M, int64_t N) {
     int64_t tile = 0;
     q8_tile_nt(M, N, &tile);
@@ -910,9 +911,9 @@ static int packed_gemm(const int8_t* a, const float* a_s, int64_t as_sm, const i
     const bool can_stream = M >= 1 && M <= 16 && (N / 16) * (K / 64) < ((int64_t)1 << 31) &&
                             M * K < ((int64_t)1 << 31) && workspace &&
                             workspace_bytes >= q8_stream_workspace_bytes(N, K);
-    // by default: the balanced kernel up to 16 rows (given its workspace), the row-round decode kernel up to 64 rows
-    // (and up to 16 without a workspace), beyond them the register-fold kernel or the tile kernel
-    if (kernel == -1) kernel = M >= 1 && M <= 16 && can_stream ? 4 : M <= 64 ? 1 : q8_mid_faster(M, N) ? 2 : 0;
+    // by default up to 16 rows the balanced kernel given its workspace, else the row-round decode kernel; beyond them the
+    // register-fold kernel or the tile kernel
+    if (kernel == -1) kernel = M >= 1 && M <= 16 && can_stream ? 4 : M <= 16 ? 1 : q8_mid_faster(M, N) ? 2 : 0;
     if (kernel == 0 && K > (1 << 23)) kernel = 2;      // the tile kernel's offsets within a tile are 32-bit; same bits
     if (kernel == 1 && M > 64) return PRISM_ERR_ARG;
     if (kernel == 4 && !can_stream) return M > 16 ? PRISM_ERR_SHAPE : PRISM_ERR_ARG;
