@@ -158,7 +158,8 @@ __global__ __launch_bounds__(kQThreads) void quant_rows_groups_slow_kernel(const
 }
 
 // ---------------------------------------------------------------------------------------------- rows_g (W4A8)
-// GROUP_ROW: one scale for the whole row (group == K); otherwise one per 256 inputs (32 chunks = half a wave).
+// GROUP_ROW: one scale for the whole row (group == K), one workgroup per row; otherwise one per 256 inputs (32 chunks =
+// half a wave), which need nothing of each other: a row goes over gridDim.y workgroups of NCH x 2048 inputs.
 template <int NCH, bool GROUP_ROW>
 __global__ __launch_bounds__(kQThreads) void quant_rows_g_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                  int8_t* __restrict__ xq, float* __restrict__ a,
@@ -167,17 +168,17 @@ __global__ __launch_bounds__(kQThreads) void quant_rows_g_kernel(const uint16_t*
     __shared__ float red[kQThreads / kWave];
     kernel_args_now(x, ldx, xq, a, xs, n_rows, M, K);
     const int64_t row = blockIdx.x;
-    const int nch = K / 8;
+    const int nch = K / 8, c0 = GROUP_ROW ? 0 : blockIdx.y * NCH;
     const v4u* xr = reinterpret_cast<const v4u*>(x + row * ldx);
     float v[NCH][8];
     float amax[NCH];
     float rmax = 0.f;
     v4u raw[NCH];                                      // all loads first (see rows_q8)
 #pragma unroll
-    for (int c = 0; c < NCH; c++) raw[c] = __builtin_nontemporal_load(xr + min((int)threadIdx.x + c * kQThreads, nch - 1));
+    for (int c = 0; c < NCH; c++) raw[c] = __builtin_nontemporal_load(xr + min((int)threadIdx.x + (c + c0) * kQThreads, nch - 1));
 #pragma unroll
     for (int c = 0; c < NCH; c++) {
-        const int idx = threadIdx.x + c * kQThreads;
+        const int idx = threadIdx.x + (c + c0) * kQThreads;
         amax[c] = 0.f;
         unpack_bf16x8(raw[c], v[c]);
         if (idx < nch) {
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(kQThreads) void quant_rows_g_kernel(const uint16_t*
     v2u* qr = reinterpret_cast<v2u*>(xq + row * K);
 #pragma unroll
     for (int c = 0; c < NCH; c++) {
-        const int idx = threadIdx.x + c * kQThreads;   // all lanes of a half-wave share the validity of idx
+        const int idx = threadIdx.x + (c + c0) * kQThreads;   // all lanes of a half-wave share the validity of idx
         float gmax = rmax;
         if (!GROUP_ROW) {
             gmax = amax[c];
@@ -283,15 +284,17 @@ extern "C" int prism_quant_rows_g(const uint16_t* x, int64_t ldx, int8_t* xq, fl
     const int need = (int)((K / 8 + kQThreads - 1) / kQThreads);
     dim3 grid((unsigned)M);
     const bool row = group == K && K != 256;
+    if (!row) {
+        // one workgroup per 2048 inputs, so that a long row is not one workgroup's serial work: 1 x 17408 11.8 -> 2.4 us, 100 x
+        // 17408 12.8 -> 3.4, 4096 x 17408 186 -> 64; 2048 x 5120 12.0 -> 11.8, 4096 x 2048 8.8 -> 9.1
+        hipLaunchKernelGGL((quant_rows_g_kernel<1, false>), dim3((unsigned)M, (unsigned)need), dim3(kQThreads), 0, st, x,
+                           ldx, xq, a, xs, n_rows, (int)M, (int)K);
+        PRISM_LAUNCH_CHECK();
+        return PRISM_OK;
+    }
 #define QG(N)                                                                                                       \
-    do {                                                                                                            \
-        if (row)                                                                                                    \
-            hipLaunchKernelGGL((quant_rows_g_kernel<N, true>), grid, dim3(kQThreads), 0, st, x, ldx, xq, a, xs,    \
-                               n_rows, (int)M, (int)K);                                                             \
-        else                                                                                                        \
-            hipLaunchKernelGGL((quant_rows_g_kernel<N, false>), grid, dim3(kQThreads), 0, st, x, ldx, xq, a, xs,   \
-                               n_rows, (int)M, (int)K);                                                             \
-    } while (0)
+    hipLaunchKernelGGL((quant_rows_g_kernel<N, true>), grid, dim3(kQThreads), 0, st, x, ldx, xq, a, xs, n_rows,     \
+                       (int)M, (int)K)
     if (need <= 1) QG(1);
     else if (need <= 2) QG(2);
     else if (need <= 4) QG(4);
