@@ -98,16 +98,23 @@ def _check_device(dev):
 
 def stream_of(t):
     """torch's current stream handle on t's device."""
-    idx = _check_device(t.device)
-    return ctypes.c_void_p(torch.cuda.current_stream(idx).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(_check_device(t.device))
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_fns = {}
 
 
 def call(name, *args):
-    rc = getattr(lib(), name)(*args)
+    # plain ints for the pointers and the stream (argtypes convert them in C) and the function looked up once: a
+    # decode-size call is bound by this path
+    f = _fns.get(name)
+    if f is None:
+        f = _fns[name] = getattr(lib(), name)
+    rc = f(*args)
     if rc != 0:
         msg = lib().prism_error_string(rc).decode()
         raise PrismError(f"{name}: {msg} (code {rc})")
