@@ -156,11 +156,11 @@ PRISM_API int64_t prism_w8a8_pc_split_workspace_bytes(int64_t M, int64_t N);
  * Q8_0 W8A8 GEMM (gk = 32, one activation scale per token) on packed weights: the arithmetic and bits of
  * prism_w8a8_gemm with gk = 32 (kernels/w8a8.py:64-85), the engine entry kernels/w8a8.py:183-231.
  * a int8 [M, K]; a_s fp32, row m at a_s[m * as_sm]; qt / dt from prism_q8_0_pack; out as prism_w8a8_gemm.
- * kernel: -1 picks by M; 0 the prefill tile kernel; 1 the decode kernels (M <= 64: M <= 16 folds through LDS,
+ * kernel: -1 picks by shape; 0 the prefill tile kernel; 1 the decode kernels (M <= 64: M <= 16 folds through LDS,
  * larger M as kernel 2); 2 the register-fold kernel, one wave per 16 x 16 output tile (any M up to 65535 x 16: the
  * choice for narrow projections, whose few 128 x 128 tiles leave CUs idle); 3 the prefill tile kernel in a
  * reassociated order that is not the reference's: per block y = fma(float(P), sw, y), then y = RN(y a_s[m]) (the
- * per-token scale factored out of the block sum), half the epilogue's vector work.  Kernel 3's bf16 outputs equal
+ * per-token scale factored out of the block sum), two instructions per output and block for three (K <= 2^23).  Kernel 3's bf16 outputs equal
  * kernel 0's on all but a few in 10^4 outputs and are within 1 bf16 ulp plus 2 (K/32 + 2) 2^-24 sum |terms| of them.
  * 4 the balanced decode kernel (1 <= M <= 16): min(N/16, 256) workgroups take equal shares of the projection's
  * 1 KB weight chunks, so every CU streams the same bytes; a 16-row tile split between two workgroups hands its
@@ -172,7 +172,7 @@ PRISM_API int64_t prism_w8a8_pc_split_workspace_bytes(int64_t M, int64_t N);
  * (csrc/w8a8_gemm.cu:794-797), which its engine allocates once per device (kernels/cuda_ext.py:138-143).
  * Bytes past the first 512 KB (the most any shape's handoff words take) are scratch for the tile kernels (0, 3):
  * from M >= 1024 on N >= 16384, where they hold ceil(M / 128) 128 K bytes, the activations are first copied there as
- * 128-row panels (each 128-input stage of a tile in one 16 KB piece); same bits, about 1% faster at config 1.
+ * panels (32 rows x 32 inputs, a wave's MFMA operand, in one 1 KB piece); same bits.
  * Needs K % 128 == 0.
  */
 PRISM_API int prism_w8a8_q8_0_packed_gemm(const int8_t* a, const float* a_s, int64_t as_sm, const int8_t* qt,

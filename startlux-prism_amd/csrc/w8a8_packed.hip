@@ -240,12 +240,7 @@ __global__ __launch_bounds__((NW + FW) * 64) void w8a8_packed_decode_kernel(cons
 }
 
 // ---------------------------------------------------------------------------------------------- prefill tile
-// 128 x 128 output tile per 256-thread workgroup (2 x 2 waves of 64 x 64), v_mfma_i32_32x32x32_i8 per (32 x 32,
-// block), 4 blocks (2 chunk pairs) per stage.  The weight tile of a stage is 8 tiles x 2 chunks = 8 runs of 2 KB,
-// copied to LDS as they are; a B fragment (column n, 16 bytes of a block) is two 8-byte pieces of a chunk.
-constexpr int PBM = 128, PBN = 128;
-constexpr int PLDA = 128 + 16;          // activation tile row (bytes), padded
-constexpr int PLDB = 2048 + 64;         // one 16-row tile's two chunks, padded
+constexpr int PBM = 128;
 
 // The exact-order prefill tile: 128 x 32 NT outputs per 256-thread workgroup, each wave 32 activation rows x 32 NT columns
 // (NT v_mfma_i32_32x32x32_i8 per block), stages of 4 blocks (2 chunk pairs).  The VALU bounds it:
@@ -261,9 +256,14 @@ constexpr int PLDB = 2048 + 64;         // one 16-row tile's two chunks, padded
 //   * all of a wave's outputs lie on the same 32 rows: a lane holds the scaled activation scale and offset of 16 rows
 //     (32 registers; 64 if it held 64 x 64 outputs), and the activation fragments, which no other wave of an m-row
 //     needs, come straight from memory into the registers the MFMA reads, each block's a stage ahead.
+// Measured with the panel copy at 8192 x 27648 x 5120: 3.84-3.88 ms (conversion and four dependent instructions per output
+// and block, both operands through single-buffered LDS) -> 2.94-3.02 ms; 777 x 13824 x 5120: 254-262 -> 175-179 us.
+// RA: the reassociated order (one activation scale per token, factored out of the block sum): per block
+// y = fma(float(P), sw, y), then y = RN(y sa) once after the K loop; two instructions per output and block (2.80-2.85 ->
+// 2.51 ms and 201 -> 157 us).
 // Waves with no live row only stage the weights and keep the barriers.  PAN: `a` is the panel copy of
 // q8_act_panel_kernel, a fragment one 1 KB piece; otherwise it is 32 rows' 32 bytes.
-template <int EPI, bool PAN, int NT>
+template <int EPI, bool PAN, int NT, bool RA = false>
 __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __restrict__ a,
                                                                 const float* __restrict__ a_s, int64_t as_sm,
                                                                 const int8_t* __restrict__ qt,
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
         ok = ok && q8_scale_ok(sa[r]);
     }
     gload(0);
-    const bool all_ok = __syncthreads_and(ok);
+    const bool all_ok = RA || __syncthreads_and(ok);
     load_a(0, 0);                                    // in the loop's own order, so that its waits can be as late
     load_a(0, 1);
     store();
@@ -415,13 +415,17 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
                 float p[16];
 #pragma unroll
                 for (int r = 0; r < 16; r++)
-                    p[r] = PLAIN ? mul_rn((float)acc[s & 1][r], sa[r]) : q8_term(acc[s & 1][r], sa[r], sc[r]);
+                    p[r] = RA ? (float)acc[s & 1][r]
+                              : PLAIN ? mul_rn((float)acc[s & 1][r], sa[r]) : q8_term(acc[s & 1][r], sa[r], sc[r]);
                 __builtin_amdgcn_sched_barrier(0);
+                if (!RA) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) p[r] = mul_rn(p[r], sw[s & 3]);
-                __builtin_amdgcn_sched_barrier(0);
+                    for (int r = 0; r < 16; r++) p[r] = mul_rn(p[r], sw[s & 3]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
 #pragma unroll
-                for (int r = 0; r < 16; r++) y[s % NT][r] = add_rn(y[s % NT][r], p[r]);
+                for (int r = 0; r < 16; r++)
+                    y[s % NT][r] = RA ? __builtin_fmaf(p[r], sw[s & 3], y[s % NT][r]) : add_rn(y[s % NT][r], p[r]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -433,8 +437,14 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
         }
     };
     // every wave of the workgroup takes the same loop (the barriers are in it)
-    if (all_ok) loop(std::false_type{});
+    if (!RA && all_ok) loop(std::false_type{});
     else loop(std::true_type{});
+    if (RA) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) y[t][r] = mul_rn(y[t][r], sa[r]);
+    }
 #pragma unroll
     for (int t = 0; t < NT; t++) {
         const int n = n0 + swc + 32 * t;
@@ -452,162 +462,6 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
             }
         }
     }
-}
-
-// RA: the reassociated order (one activation scale per token, factored out of the block sum): per block
-// y = fma(float(P), sw, y), then y = RN(y sa) once; 2 VALU operations per output and block instead of 4.
-// PAN: `a` is the panel copy of q8_act_panel_kernel.
-template <int EPI, bool PAN = false>
-__global__ __launch_bounds__(256, 2) void w8a8_packed_reassoc_kernel(const int8_t* __restrict__ a,
-                                                                  const float* __restrict__ a_s, int64_t as_sm,
-                                                                  const int8_t* __restrict__ qt,
-                                                                  const uint16_t* __restrict__ dt,
-                                                                  void* __restrict__ out, int64_t ldo,
-                                                                  const int32_t* __restrict__ n_rows, int M, int N,
-                                                                  int K, int tiles_m, int tiles_n) {
-    __shared__ __attribute__((aligned(16))) int8_t As[PBM * PLDA];
-    __shared__ __attribute__((aligned(16))) int8_t Bs[8 * PLDB];
-    __shared__ float sws[4][PBN];
-
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wm = wv >> 1, wn = wv & 1;
-    int pm, pn;
-    xcd_tile_coords(blockIdx.x, tiles_m, tiles_n, pm, pn);
-    const int m0 = pm * PBM, n0 = pn * PBN;
-    const int live = min(M, __ldg(n_rows));
-    if (m0 >= live) return;
-    const int G = K / 32, KP = K / 64;
-    const int nt0 = n0 / 16, ntiles = N / 16;
-
-    // activation loader: chunk i = row lr + 32 i, bytes lc .. lc + 15 of the stage's 128 bytes
-    const int lr = tid >> 3, lc = (tid & 7) * 16;
-    const int8_t* ap[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        if (PAN) {                                   // the panel of row group m0 / 32 + i: row lr, the stage's bytes lc ..
-            ap[i] = a + (int64_t)(m0 + 32 * i) * K + (lc >> 5) * 1024 + ((lc >> 4) & 1) * 512 + lr * 16;
-        } else {
-            ap[i] = a + (int64_t)min(m0 + lr + 32 * i, M - 1) * K + lc;
-        }
-    }
-    // weight loader: chunk c = tid + 256 i -> tile c / 128 (clamped in range), 16 bytes (c % 128) of its 2 KB run
-    const v4i* bp[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int c = tid + 256 * i;
-        const int t = min(nt0 + (c >> 7), ntiles - 1);
-        bp[i] = reinterpret_cast<const v4i*>(qt) + (int64_t)t * KP * 64 + (c & 127);
-    }
-    // scale loader: thread t < 64 -> tile t / 8, 16 bytes (t % 8) of the tile's 2 x 64 bytes (2 pairs)
-    const int st_t = min(nt0 + (tid >> 3), ntiles - 1);
-    const v4u* sp = reinterpret_cast<const v4u*>(dt) + (int64_t)st_t * KP * 4 + (tid & 7);
-
-    v4i ra[4], rb[4];
-    v4u rs;
-    auto gload = [&](int kb) {                       // kb: first block of the stage (a multiple of 4)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            ra[i] = *reinterpret_cast<const v4i*>(ap[i] + (PAN ? (int64_t)kb * 1024 : (int64_t)kb * 32));
-            rb[i] = __builtin_nontemporal_load(bp[i] + (int64_t)(kb / 2) * 64);
-        }
-        rs = sp[(int64_t)(kb / 2) * 4];
-    };
-
-    const int lrow = 4 * (lane >> 5);
-    float sa[2][16];
-    auto load_sa = [&]() {
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = min(m0 + wm * 64 + mt * 32 + 8 * (r >> 2) + lrow + (r & 3), M - 1);
-                sa[mt][r] = a_s[(int64_t)m * as_sm];
-            }
-    };
-    float y[2][2][16];
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) y[mt][nt][r] = 0.f;
-
-    const int arow0 = (wm * 64 + (lane & 31)) * PLDA + (lane >> 5) * 16;
-    // B fragment of column j = wn * 64 + nt * 32 + lane % 32 (tile-local), lane group g = lane / 32: pieces
-    // q = 2 g and 2 g + 1 of row j % 16 in 16-row tile j / 16
-    int bofs[2];
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const int j = wn * 64 + t * 32 + (lane & 31);
-        bofs[t] = (j >> 4) * PLDB + ((j & 15) + 32 * (lane >> 5)) * 16;
-    }
-    const int swc = wn * 64 + (lane & 31);
-    const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    gload(0);
-    for (int kb = 0; kb < G; kb += 4) {
-        lds_barrier();
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int c = tid + 256 * i;
-            *reinterpret_cast<v4i*>(&As[(lr + 32 * i) * PLDA + lc]) = ra[i];
-            *reinterpret_cast<v4i*>(&Bs[(c >> 7) * PLDB + (c & 127) * 16]) = rb[i];
-        }
-        if (tid < 64) {
-            // rs: tile tid / 8, pair (tid % 8) / 4, rows 4 ((tid % 8) % 4) .. +3, both blocks of the pair
-            const int tl = tid >> 3, pr = (tid & 7) >> 2, r0 = 4 * (tid & 3);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                sws[2 * pr][16 * tl + r0 + e] = f16_to_f32(rs[e] & 0xffffu);
-                sws[2 * pr + 1][16 * tl + r0 + e] = f16_to_f32(rs[e] >> 16);
-            }
-        }
-        lds_barrier();
-        if (kb + 4 < G) gload(kb + 4);
-#pragma unroll
-        for (int bi = 0; bi < 4; bi++) {
-            v4i fa[2], fb[2];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                fa[t] = *reinterpret_cast<const v4i*>(&As[arow0 + t * 32 * PLDA + bi * 32]);
-                const int o = bofs[t] + (bi >> 1) * 1024 + 8 * (bi & 1);
-                const int64_t p0 = *reinterpret_cast<const int64_t*>(&Bs[o]);
-                const int64_t p1 = *reinterpret_cast<const int64_t*>(&Bs[o + 16 * 16]);
-                fb[t] = v4i{(int)p0, (int)(p0 >> 32), (int)p1, (int)(p1 >> 32)};
-            }
-            const float sw[2] = {sws[bi][swc], sws[bi][swc + 32]};
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                for (int nt = 0; nt < 2; nt++) {
-                    const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[mt], fb[nt], zero, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        y[mt][nt][r] = __builtin_fmaf((float)acc[r], sw[nt], y[mt][nt][r]);
-                    }
-                }
-        }
-    }
-    load_sa();                                       // the scales, applied once after the K loop
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            const int n = n0 + wn * 64 + nt * 32 + (lane & 31);
-            if (n >= N) continue;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + wm * 64 + mt * 32 + 8 * (r >> 2) + lrow + (r & 3);
-                if (m < live) {
-                    y[mt][nt][r] = mul_rn(y[mt][nt][r], sa[mt][r]);
-                    if (EPI == 0) {
-                        reinterpret_cast<uint16_t*>(out)[(int64_t)m * ldo + n] = (uint16_t)f32_to_bf16(y[mt][nt][r]);
-                    } else {
-                        float* o = reinterpret_cast<float*>(out) + (int64_t)m * ldo + n;
-                        *o = add_rn(*o, y[mt][nt][r]);
-                    }
-                }
-            }
-        }
 }
 
 // ---------------------------------------------------------------------------------------------- mid
@@ -853,8 +707,8 @@ static void launch_packed(int kernel, const int8_t* a, const float* a_s, int64_t
                            n_rows, M, N, K, tiles_m, tiles_n);                                                     \
     } while (0)
         if (kernel == 3) {
-            if (pan) Q8T((w8a8_packed_reassoc_kernel<EPI, true>), PBN);
-            else Q8T((w8a8_packed_reassoc_kernel<EPI, false>), PBN);
+            if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 4, true>), 128);
+            else Q8T((w8a8_q8_tile_kernel<EPI, false, 4, true>), 128);
         } else {
             int64_t cost = 0;
             const int nt = q8_tile_nt(M, N, &cost);
@@ -915,6 +769,7 @@ static int packed_gemm(const int8_t* a, const float* a_s, int64_t as_sm, const i
     // register-fold kernel or the tile kernel
     if (kernel == -1) kernel = M >= 1 && M <= 16 && can_stream ? 4 : M <= 16 ? 1 : q8_mid_faster(M, N) ? 2 : 0;
     if (kernel == 0 && K > (1 << 23)) kernel = 2;      // the tile kernel's offsets within a tile are 32-bit; same bits
+    if (kernel == 3 && K > (1 << 23)) return PRISM_ERR_SHAPE;
     if (kernel == 1 && M > 64) return PRISM_ERR_ARG;
     if (kernel == 4 && !can_stream) return M > 16 ? PRISM_ERR_SHAPE : PRISM_ERR_ARG;
     if (kernel == 2 && M > 65535 * 16) return PRISM_ERR_SHAPE;         // grid rows: one per 16 activation rows
