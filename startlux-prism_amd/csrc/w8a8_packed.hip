@@ -17,6 +17,7 @@
 
 #include "common.h"
 #include "q8_stream.h"
+#include "q8_tile_src.h"
 
 
 namespace prism {
@@ -283,33 +284,22 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
     const int m0 = pm * PBM, n0 = pn * BN;
     const int live = min(M, __ldg(n_rows));
     if (m0 >= live) return;
-    const int KP = K / 64, NS = K / 128;
-    const int nt0 = n0 / 16, ntiles = N / 16;
+    const int NS = K / 128;
 
-    // Buffer loads, each operand's tile base in SGPRs and the stage's offset in soffset, so the loop computes no
-    // addresses; the record counts end with the operands, so rows past M or N read zeros.  Activations: lane l's 16
-    // bytes of a block are row l % 32, inputs 16 (l / 32) .. + 15.
+    // buffer loads: each operand's base in SGPRs and the stage's offset in soffset, so the loop computes no addresses
+    const Q8TileSrc<NT> src = q8_tile_src<PAN, NT>(m0, n0, wv, lane, M, N, K);
     const int mw = m0 + 32 * wv;                     // the wave's first row
-    const auto ar = PAN ? buf_rsrc(a + (int64_t)mw * K)
-                        : buf_rsrc_n(a + (int64_t)min(mw, M - 1) * K,
-                                     (uint32_t)min((int64_t)max(M - mw, 0) * K, (int64_t)0x7fffffff));
-    const uint32_t av = PAN ? lane * 16 : (lane & 31) * K + (lane >> 5) * 16;
-    // weights: chunk c = tid + 256 i -> tile c / 128, 16 bytes (c % 128) of its 2 KB run
-    const auto br = buf_rsrc_n(qt + (int64_t)nt0 * KP * 1024,
-                               (uint32_t)min((int64_t)(ntiles - nt0) * KP * 1024, (int64_t)0x7fffffff));
-    const uint32_t bv = (uint32_t)(tid >> 7) * KP * 1024 + (tid & 127) * 16;
-    // scales: thread -> tile tid / 32 (past the 2 NT: not read), pair (tid / 16) % 2, row tid % 16: both blocks' fp16
-    const auto sr = buf_rsrc_n(dt + (int64_t)nt0 * KP * 32,
-                               (uint32_t)min((int64_t)(ntiles - nt0) * KP * 64, (int64_t)0x7fffffff));
-    const uint32_t sv = (uint32_t)(tid >> 5) * KP * 64 + (tid & 31) * 4;
+    const auto ar = buf_rsrc(a + src.a_base);
+    const auto br = buf_rsrc(qt + src.w_base);
+    const auto sr = buf_rsrc(reinterpret_cast<const int8_t*>(dt) + src.s_base);
 
     v4i rb[NT];
     uint32_t rs;
     auto gload = [&](int st) {                       // past the end: the last stage again
         st = min(st, NS - 1);
 #pragma unroll
-        for (int i = 0; i < NT; i++) rb[i] = buf_load16<kBufNT>(br, bv, st * 2048 + i * 2 * KP * 1024);
-        rs = buf_load4(sr, sv, st * 128);
+        for (int i = 0; i < NT; i++) rb[i] = buf_load16<kBufNT>(br, src.w_v, src.w_s[i] + st * 2048);
+        rs = buf_load4(sr, src.s_v, st * 128);
     };
     // A weight stage is stored block by block, [16-row tile][pair][block of the pair][q / 2][row][q % 2] of 8 bytes, so
     // that a B fragment (below) is one 16-byte read, 16 lanes of it 256 contiguous bytes (no bank conflict).
@@ -330,7 +320,7 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
 
     v4i fa[4];                                       // the wave's fragment of each block of a stage
     auto load_a = [&](int st, int bi) {              // past the end: the last stage again
-        fa[bi] = buf_load16(ar, av, PAN ? min(st, NS - 1) * 4096 + bi * 1024 : min(st, NS - 1) * 128 + bi * 32);
+        fa[bi] = buf_load16(ar, src.a_v, PAN ? min(st, NS - 1) * 4096 + bi * 1024 : min(st, NS - 1) * 128 + bi * 32);
     };
 
     const int lrow = 4 * (lane >> 5);
