@@ -77,7 +77,7 @@ __device__ __forceinline__ float mul_f16_rn(float x, uint32_t word) {
 // Nothing under- or overflows differently while 2^-48 <= |sa| < 2^31 or sa = 0 (q8_scale_ok; a quantizer's scale is at
 // least 1e-10 / 127 > 2^-41): every nonzero |P sa sw| 2^-53 is then a normal fp32 (fp16 |sw| >= 2^-24), and an fp32 sum
 // of K / 32 <= 2^25 terms below 2^66 stays far from 2^128.  Zeros may differ in sign, which the running sum (never -0)
-// cannot show.  Rows outside the range take the plain fold.
+// cannot show.  A tile with a live row outside the range takes the plain fold.
 constexpr int kQ8Bias = 1 << 19;
 __device__ __forceinline__ bool q8_scale_ok(float sa) {
     const uint32_t e = (__float_as_uint(sa) >> 23) & 0xff;               // zero, or 127 - 48 <= e < 127 + 31

@@ -326,9 +326,10 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
     const int lrow = 4 * (lane >> 5);
     float sa[16], sc[16];
     bool ok = true;
+    // past the live rows: the last live row's scale (a bucket's own may be stale, and must not cost the tile its fold)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-        sa[r] = a_s[(int64_t)min(mw + 8 * (r >> 2) + lrow + (r & 3), M - 1) * as_sm];
+        sa[r] = a_s[(int64_t)min(mw + 8 * (r >> 2) + lrow + (r & 3), live - 1) * as_sm];
         ok = ok && q8_scale_ok(sa[r]);
     }
     gload(0);
