@@ -160,7 +160,7 @@ PRISM_API int64_t prism_w8a8_pc_split_workspace_bytes(int64_t M, int64_t N);
  * larger M as kernel 2); 2 the register-fold kernel, one wave per 16 x 16 output tile (any M up to 65535 x 16: the
  * choice for narrow projections, whose few 128 x 128 tiles leave CUs idle); 3 the prefill tile kernel in a
  * reassociated order that is not the reference's: per block y = fma(float(P), sw, y), then y = RN(y a_s[m]) (the
- * per-token scale factored out of the block sum), two instructions per output and block for three (K <= 2^23).  Kernel 3's bf16 outputs equal
+ * per-token scale factored out of the block sum), two instructions per output and block for three.  Kernel 3's bf16 outputs equal
  * kernel 0's on all but a few in 10^4 outputs and are within 1 bf16 ulp plus 2 (K/32 + 2) 2^-24 sum |terms| of them.
  * 4 the balanced decode kernel (1 <= M <= 16): min(N/16, 256) workgroups take equal shares of the projection's
  * 1 KB weight chunks, so every CU streams the same bytes; a 16-row tile split between two workgroups hands its

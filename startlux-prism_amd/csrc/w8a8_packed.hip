@@ -467,8 +467,8 @@ __global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __re
 // lanes' pieces into the operand layout of the weight chunk (lane q: bytes 8q..8q+7 of each block).  Loading the
 // activation rows in 64-byte runs instead of eight-byte pieces halved this kernel's time.  Each block's int32 sums
 // come from one v_mfma_i32_16x16x32_i8 with a zero accumulator and the lane folds RN(RN(float(P) sa) sw) into its
-// outputs in block order, in registers.
-template <int PD, int MT, int TG, int EPI>
+// outputs in block order, in registers.  RA: the reassociated order of the tile kernel (for K beyond its 32-bit offsets).
+template <int PD, int MT, int TG, int EPI, bool RA = false>
 __global__ __launch_bounds__(64) void w8a8_packed_mid_kernel(const int8_t* __restrict__ a,
                                                               const float* __restrict__ a_s, int64_t as_sm,
                                                               const int8_t* __restrict__ qt,
@@ -544,6 +544,11 @@ __global__ __launch_bounds__(64) void w8a8_packed_mid_kernel(const int8_t* __res
                 for (int t = 0; t < MT; t++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
+                        if (RA) {
+                            const float sw = f16_to_f32(h ? p.s[g] >> 16 : p.s[g] & 0xffffu);
+                            y[g][t][e] = __builtin_fmaf((float)acc[g][t][h][e], sw, y[g][t][e]);
+                            continue;
+                        }
                         const float x = mul_rn((float)acc[g][t][h][e], sa[t][e]);
                         y[g][t][e] = add_rn(y[g][t][e], h ? mul_f16_rn<1>(x, p.s[g]) : mul_f16_rn<0>(x, p.s[g]));
                     }
@@ -584,6 +589,7 @@ __global__ __launch_bounds__(64) void w8a8_packed_mid_kernel(const int8_t* __res
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int row = m0 + 16 * t + 4 * q + e;
+                if (RA) y[g][t][e] = mul_rn(y[g][t][e], sa[t][e]);
                 if (row < live) {
                     if (EPI == 0) {
                         reinterpret_cast<uint16_t*>(out)[(int64_t)row * ldo + n] = (uint16_t)f32_to_bf16(y[g][t][e]);
@@ -667,6 +673,11 @@ static void launch_packed(int kernel, const int8_t* a, const float* a_s, int64_t
         else kernel = 2;
 #undef PDEC_
 #undef PDEC
+    }
+    if (kernel == 3 && K > (1 << 23)) {              // the tile kernel's offsets within a tile are 32-bit
+        hipLaunchKernelGGL((w8a8_packed_mid_kernel<8, 1, 1, EPI, true>), dim3(N / 16, (M + 15) / 16), dim3(64), 0, st,
+                           a, a_s, as_sm, qt, dt, out, ldo, n_rows, M, N, K);
+        return;
     }
     if (kernel == 2) {
         // from 33 rows: each wave one m-tile and two weight tiles (one activation request serves both; the same wave
@@ -760,10 +771,10 @@ static int packed_gemm(const int8_t* a, const float* a_s, int64_t as_sm, const i
     // register-fold kernel or the tile kernel
     if (kernel == -1) kernel = M >= 1 && M <= 16 && can_stream ? 4 : M <= 16 ? 1 : q8_mid_faster(M, N) ? 2 : 0;
     if (kernel == 0 && K > (1 << 23)) kernel = 2;      // the tile kernel's offsets within a tile are 32-bit; same bits
-    if (kernel == 3 && K > (1 << 23)) return PRISM_ERR_SHAPE;
     if (kernel == 1 && M > 64) return PRISM_ERR_ARG;
     if (kernel == 4 && !can_stream) return M > 16 ? PRISM_ERR_SHAPE : PRISM_ERR_ARG;
-    if (kernel == 2 && M > 65535 * 16) return PRISM_ERR_SHAPE;         // grid rows: one per 16 activation rows
+    if ((kernel == 2 || (kernel == 3 && K > (1 << 23))) && M > 65535 * 16)
+        return PRISM_ERR_SHAPE;                                        // grid rows: one per 16 activation rows
     if (M == 0) return PRISM_OK;
     hipStream_t st = (hipStream_t)stream;
     if (kernel == 4) {
@@ -776,8 +787,8 @@ static int packed_gemm(const int8_t* a, const float* a_s, int64_t as_sm, const i
     // the tile kernels on a panel copy of the activations where the workspace holds it past the handoff words and the
     // shape repays the copy (2 M K bytes of traffic): from 1024 rows on projections at least 16384 wide
     int8_t* pan = nullptr;
-    if ((kernel == 0 || kernel == 3) && M >= 1024 && N >= 16384 && M <= 8191 * 128 && workspace &&
-        PRISM_ALIGNED(workspace, 256) && workspace_bytes >= kQ8PanelOffset + (M + 127) / 128 * 128 * K)
+    if ((kernel == 0 || kernel == 3) && K <= (1 << 23) && M >= 1024 && N >= 16384 && M <= 8191 * 128 &&
+        workspace && PRISM_ALIGNED(workspace, 256) && workspace_bytes >= kQ8PanelOffset + (M + 127) / 128 * 128 * K)
         pan = static_cast<int8_t*>(workspace) + kQ8PanelOffset;
     if (epi == 0)
         launch_packed<0>(kernel, a, a_s, as_sm, qt, dt, out, ldo, n_rows, (int)M, (int)N, (int)K, st, pan);

@@ -37,6 +37,8 @@ def test_q8_0_packed_gemm_checks(lib):
     assert call(kernel=1, M=65) == ARG           # the decode kernels hold up to 64 rows
     assert call(M=0) == OK
     assert call(M=0, kernel=3) == OK             # the reassociated prefill kernel is a valid choice
+    assert call(M=0, kernel=3, K=(1 << 23) + 128) == OK          # ... of any K the exact kernels take
+    assert call(M=0, kernel=0, K=(1 << 23) + 128) == OK
 
 
 def test_pack_checks_match_the_gemms(lib):

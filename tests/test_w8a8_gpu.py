@@ -339,6 +339,19 @@ def test_packed_reassoc_bit_exact(dev, M, N, K, live):
     assert np.array_equal(got1, want1)
 
 
+@pytest.mark.parametrize("kernel", ["reassoc", "tile"])
+def test_packed_tile_long_k(dev, kernel):
+    """K beyond the tile kernel's 32-bit offsets (2^23): both of its orders are still taken, with the same bits."""
+    M, N, K, live = 18, 16, (1 << 23) + 128, 17
+    g = rng(K)
+    qs, a = (g.integers(-127, 128, (r, K), dtype=np.int8) for r in (N, M))
+    d = (g.random((N, K // 32)) * 1e-3).astype(np.float16).view(np.uint16)
+    s = (g.random(M) * 1e-2).astype(np.float32)
+    want = (O.w8a8_gemm_reassoc if kernel == "reassoc" else O.w8a8_gemm)(a, s, qs, d, 32, epi=0, live=live)
+    got = _packed_gemm(dev, a, s, qs, d, 0, kernel, live=live).view(torch.int16).cpu().numpy().view(np.uint16)
+    assert np.array_equal(got[:live], want[:live]) and (got[live:] == 7).all()
+
+
 def test_reassoc_only_for_packed_q8(dev):
     from prism_amd import w8a8 as KW
     a = torch.zeros(4, 128, dtype=torch.int8, device=dev)
