@@ -98,7 +98,12 @@ def _check_device(dev):
 
 def stream_of(t):
     """torch's current stream handle on t's device."""
-    return torch._C._cuda_getCurrentRawStream(_check_device(t.device))
+    return raw_stream(_check_device(t.device))
+
+
+def raw_stream(idx):
+    """torch's current stream handle on device idx."""
+    return torch._C._cuda_getCurrentRawStream(idx)
 
 
 def ptr(t):

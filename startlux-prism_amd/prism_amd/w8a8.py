@@ -25,11 +25,12 @@ import torch
 
 from . import _lib as L
 from . import dispatch
+from . import scratch
 from .quant import quant_rows  # noqa: F401  (re-exported: kernels/w8a8.py:264)
 
 KERNELS = {"auto": -1, "tile": 0, "decode": 1, "mid": 2, "reassoc": 3, "stream": 4}
 # "stream" (packed Q8_0, 1..16 rows): the balanced decode kernel, whose workgroups take equal shares of the weight
-# chunks and hand a split tile's running sums on through a small per-device workspace (workspace()).
+# chunks and hand a split tile's running sums on through a small workspace (workspace()).
 # "reassoc" (packed Q8_0 only, by request, never chosen by "auto"): the prefill tile kernel with the per-token
 # activation scale factored out of the block sum (y = fma(float(P), sw, y) per block, then y * a_s once), half the
 # exact epilogue's vector work; not the reference's rounding order, so its bf16 outputs differ from the exact kernels'
@@ -190,29 +191,21 @@ def _tabled(kernel, N, K, M, gk, packed_q8=False):
     return c if ok else "auto"
 
 
-_WS = {}
 # the handoff words (the first 512 KB, the most any shape needs) and the prefill tile kernels' panel copy of the
 # activations after them (ceil(M / 128) 128 K bytes; the library takes it from 1024 rows on projections at least
 # 16384 wide)
 Q8_HANDOFF_BYTES = 512 << 10
 Q8_WS_BYTES = Q8_HANDOFF_BYTES + (96 << 20)
+_WS = scratch.Scratch(Q8_WS_BYTES, zeroed=Q8_HANDOFF_BYTES)
 
 
-def workspace(dev):
-    """The per-device workspace of the packed Q8_0 GEMM (the reference schema's `workspace`, allocated once per device
-    as kernels/cuda_ext.py:138-143 does): the "stream" kernel's handoff words, zeroed once and left zeroed by every
-    launch, then the prefill's panel copy of the activations.  None while a graph is
-    being captured on a device that has none yet (its zero fill would be a graph node): "auto" then picks another
-    kernel and "stream" raises."""
-    idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    ws = _WS.get(idx)
-    if ws is None:
-        if torch.cuda.is_current_stream_capturing():
-            return None
-        ws = torch.zeros(Q8_WS_BYTES, dtype=torch.uint8, device=torch.device("cuda", idx))
-        torch.cuda.current_stream(idx).synchronize()
-        _WS[idx] = ws
-    return ws
+def workspace(dev, panels=False):
+    """The workspace of the packed Q8_0 GEMM on dev's current stream (the reference schema's `workspace`, allocated once
+    per device as kernels/cuda_ext.py:138-143 does): the "stream" kernel's handoff words, zeroed once and left zeroed by
+    every launch, then the prefill's panel copy of the activations.  Under graph capture the words alone, or with `panels`
+    the room for the copy alone, and None on a device with no eager call yet (the words' zero fill would be a graph
+    node): "auto" then picks another kernel and "stream" raises.  See scratch.py for what calls may share."""
+    return _WS.get(dev, zeroed=not panels)
 
 
 def _gemm_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
@@ -230,35 +223,29 @@ def _gemm_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
         raise ValueError(f"out must be {want} [>= {M}, >= {w.n}] with unit column stride")
     pan = M >= 1024 and w.n >= 16384 and kernel in ("auto", "tile", "reassoc") and \
         Q8_HANDOFF_BYTES + (M + 127) // 128 * 128 * K <= Q8_WS_BYTES
-    ws = workspace(a.device) if (M <= 16 and kernel in ("auto", "decode", "stream")) or pan else None
+    ws = workspace(a.device, pan) if (M <= 16 and kernel in ("auto", "decode", "stream")) or pan else None
     if kernel == "stream" and ws is None and asked == "auto":
         kernel = "auto"             # the table's pick needs the workspace; the library then picks without it
     if kernel == "stream" and ws is None:
         raise L.PrismError('kernel "stream" needs the device workspace, made outside graph capture: run one eager '
                            'call first')
-    L.call("prism_w8a8_q8_0_packed_gemm", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt), L.ptr(w.dt), L.ptr(out),
-           out.stride(0), L.ptr(n_rows), M, w.n, K, epi, KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(),
-           L.stream_of(a))
+    # (two launches with the panels: the copy and the tile kernel that reads it)
+    scratch.call(pan, "prism_w8a8_q8_0_packed_gemm", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt), L.ptr(w.dt),
+                 L.ptr(out), out.stride(0), L.ptr(n_rows), M, w.n, K, epi, KERNELS[kernel], L.ptr(ws),
+                 0 if ws is None else ws.numel(), L.stream_of(a))
     return None
 
 
-_PCWS = {}
 PC_WS_BYTES = 96 << 20        # as the reference's workspace (kernels/cuda_ext.py:20): the split decode's slots, or
                               # the tile kernel's panel copy of the activations
+_PCWS = scratch.Scratch(PC_WS_BYTES)
 
 
 def pc_workspace(dev):
-    """The per-device workspace of the per-channel GEMM: the split decode's int32 slots (kernel "split") or the tile
-    kernel's panel copy of the activations (wide projections from 1024 rows), rewritten by every launch.  None while a graph is being captured on a device that has none yet: "auto" then picks another
-    kernel and "split" raises."""
-    idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    ws = _PCWS.get(idx)
-    if ws is None:
-        if torch.cuda.is_current_stream_capturing():
-            return None
-        ws = torch.empty(PC_WS_BYTES, dtype=torch.uint8, device=torch.device("cuda", idx))
-        _PCWS[idx] = ws
-    return ws
+    """The workspace of the per-channel GEMM on dev's current stream: the split decode's int32 slots (kernel "split") or
+    the tile kernel's panel copy of the activations (wide projections from 1024 rows), rewritten by every launch.  None
+    under graph capture on a device with no eager call yet: "auto" then picks another kernel and "split" raises."""
+    return _PCWS.get(dev)
 
 
 _PC_KERNELS = {"auto": -1, "tile": 0, "decode": 1, "split": 2}
@@ -289,9 +276,9 @@ def _gemm_pc_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
     if kernel == "split" and ws is None:
         raise L.PrismError('kernel "split" needs the device workspace, made outside graph capture: run one eager '
                            'call first')
-    L.call("prism_w8a8_pc_packed_gemm_ws", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt), L.ptr(w.ws),
-           int(w.ws.dtype == torch.float16), L.ptr(out), out.stride(0), L.ptr(n_rows), M, w.n, K, epi,
-           _PC_KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(), L.stream_of(a))
+    scratch.call(ws is not None, "prism_w8a8_pc_packed_gemm_ws", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt),
+                 L.ptr(w.ws), int(w.ws.dtype == torch.float16), L.ptr(out), out.stride(0), L.ptr(n_rows), M, w.n, K, epi,
+                 _PC_KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(), L.stream_of(a))
     return None
 
 
