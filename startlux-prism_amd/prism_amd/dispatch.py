@@ -7,7 +7,8 @@ Tables (JSON next to this module, written by prism_amd.tune on the GPU they desc
   q8_table_<tag>.json     W8A8 on Q8_0 weights (gk = 32, the packed layout): keyed and looked up as the gemm table.
                           The reference serves gk = 32 with one Triton rule and no table.
   w4a8_table_<tag>.json   W4A8: "kind,N,K" (kind q4k or q6k) -> {M: [kernel]}, looked up at the smallest measured M
-                          >= the request, else the largest (kernels/w4a8.py:309-316).
+                          >= the request, else the largest (kernels/w4a8.py:309-316); a table that ends within the
+                          decode kernels' 16 rows says nothing about more ("auto").
 <tag> is "mi355x" on gfx950.  A kernel is a name of the op's KERNELS ("tile", "decode", "mid", "stream", and "split" for the per-channel
 split decode).  STARTLUX_PRISM_GEMM_TABLE,
 STARTLUX_PRISM_Q8_TABLE and STARTLUX_PRISM_W4A8_TABLE name other files, or "off"; without a table (or for a shape it does not
@@ -69,4 +70,4 @@ def w8a8_kernel(N, K, M, gk):
 def w4a8_kernel(kind, N, K, M):
     """The table's kernel for a W4A8 product on kind ("q4k" / "q6k") weights, or "auto"."""
     entries = load("w4a8_table").get(f"{kind},{N},{K}")
-    return _at_least(entries, M) if entries else "auto"
+    return _at_least(entries, M) if entries and (M <= 16 or entries[-1][0] > 16) else "auto"

@@ -174,7 +174,7 @@ def gemm(xq, a, xs, w: W4, out, n_rows, epi=0, cfg=None, pdl=0, kernel="auto"):
     if out.dtype != want or out.shape[0] < M or out.shape[1] < w.n or out.stride(1) != 1:
         raise ValueError(f"out must be {want} [>= {M}, >= {w.n}] with unit column stride")
     if kernel == "auto":             # the MI355X table's choice for the shape, where valid (dispatch.w4a8_kernel); its
-        c = dispatch.w4a8_kernel(w.kind, w.n, K, M)      # entries end at 16 rows, beyond them the library's rule picks
+        c = dispatch.w4a8_kernel(w.kind, w.n, K, M)      # entries end at 16 rows, beyond which the library's rule picks
         ok = c == "tile" or (c in ("decode", "stream") and M <= 16)
         kernel = c if ok else "auto"
     if w.kind == "q6k":              # no mins: xs is not read

@@ -43,6 +43,17 @@ def test_w4a8_smallest_at_least(tables):
     assert dispatch.w4a8_kernel("q6k", 13824, 5120, 1) == "auto"
 
 
+def test_w4a8_decode_rows_say_nothing_about_more(tmp_path, monkeypatch):
+    """A table that ends within the decode kernels' rows, whatever its last entry: the library's rule beyond them."""
+    for last in ("tile", "decode"):
+        (tmp_path / f"{last}.json").write_text(json.dumps({"table": {"q4k,512,5120": {"4": ["decode"], "16": [last]}}}))
+        monkeypatch.setenv("STARTLUX_PRISM_W4A8_TABLE", str(tmp_path / f"{last}.json"))
+        dispatch.load.cache_clear()
+        assert dispatch.w4a8_kernel("q4k", 512, 5120, 16) == last
+        assert dispatch.w4a8_kernel("q4k", 512, 5120, 17) == "auto"
+    dispatch.load.cache_clear()
+
+
 def test_off(tables, monkeypatch):
     monkeypatch.setenv("STARTLUX_PRISM_W4A8_TABLE", "off")
     dispatch.load.cache_clear()
