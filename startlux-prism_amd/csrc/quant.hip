@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kQThreads) void quant_rows_groups_slow_kernel(const
 
 // ---------------------------------------------------------------------------------------------- rows_g (W4A8)
 // GROUP_ROW: one scale for the whole row (group == K), one workgroup per row; otherwise one per 256 inputs (32 chunks =
-// half a wave), which need nothing of each other: a row goes over gridDim.y workgroups of NCH x 2048 inputs.
+// half a wave), which need nothing of each other: a row goes over gridDim.y workgroups of NCH x 2048 inputs (prism_quant_rows_g).
 template <int NCH, bool GROUP_ROW>
 __global__ __launch_bounds__(kQThreads) void quant_rows_g_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                                  int8_t* __restrict__ xq, float* __restrict__ a,
@@ -281,17 +281,28 @@ extern "C" int prism_quant_rows_g(const uint16_t* x, int64_t ldx, int8_t* xq, fl
     if (!PRISM_ALIGNED(x, 16) || !PRISM_ALIGNED(xq, 16)) return PRISM_ERR_ALIGN;
     if (M == 0) return PRISM_OK;
     hipStream_t st = (hipStream_t)stream;
-    const int need = (int)((K / 8 + kQThreads - 1) / kQThreads);
-    dim3 grid((unsigned)M);
+    const int need = (int)((K / 8 + kQThreads - 1) / kQThreads);       // chunks of 2048 inputs in a row
     const bool row = group == K && K != 256;
     if (!row) {
-        // one workgroup per 2048 inputs, so that a long row is not one workgroup's serial work: 1 x 17408 11.8 -> 2.4 us, 100 x
-        // 17408 12.8 -> 3.4, 4096 x 17408 186 -> 64; 2048 x 5120 12.0 -> 11.8, 4096 x 2048 8.8 -> 9.1
-        hipLaunchKernelGGL((quant_rows_g_kernel<1, false>), dim3((unsigned)M, (unsigned)need), dim3(kQThreads), 0, st, x,
-                           ldx, xq, a, xs, n_rows, (int)M, (int)K);
+        // A workgroup per chunk while that does not fill the chip, so that a long row is not one workgroup's serial work (1 x
+        // 17408 11.8 -> 2.6 us, 100 x 17408 12.8 -> 3.7); beyond, up to four chunks each, a thread's loads in flight together (at one
+        // / three or four chunks: 8192 x 5120 38.1 / 29.4, 8192 x 17408 107 / 85, 8192 x 13824 88 / 71, 2048 x 8192 16.1 / 15.0; 8192 x
+        // 2560 at one / two 23.5 / 19.3).  The line: 1024 x 8192 8.1 / 8.5, 1024 x 5120 6.2 / 6.4 against 1024 x 13824 13.9 / 13.4.
+        const int parts = M <= 1024 && M * need <= 4096 ? need : (need + 3) / 4;
+        const dim3 g((unsigned)M, (unsigned)parts);
+#define QS(N)                                                                                                       \
+    hipLaunchKernelGGL((quant_rows_g_kernel<N, false>), g, dim3(kQThreads), 0, st, x, ldx, xq, a, xs, n_rows, (int)M, (int)K)
+        switch ((need + parts - 1) / parts) {
+            case 1: QS(1); break;
+            case 2: QS(2); break;
+            case 3: QS(3); break;
+            default: QS(4);
+        }
+#undef QS
         PRISM_LAUNCH_CHECK();
         return PRISM_OK;
     }
+    dim3 grid((unsigned)M);
 #define QG(N)                                                                                                       \
     hipLaunchKernelGGL((quant_rows_g_kernel<N, true>), grid, dim3(kQThreads), 0, st, x, ldx, xq, a, xs, n_rows,     \
                        (int)M, (int)K)
