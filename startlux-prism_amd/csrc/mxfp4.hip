@@ -33,8 +33,11 @@ constexpr int kMxSegSteps = 8;        // MFMA steps per accumulation segment (10
 // :110-121).  TIES == 1: nearest, ties to the even code (the OCP conversion of the C4 weights).
 template <int TIES>
 __device__ __forceinline__ uint32_t e2m1_mag(float a) {
-    if (TIES == 0)
-        return (a > .25f) + (a > .75f) + (a > 1.25f) + (a > 1.75f) + (a > 2.5f) + (a > 3.5f) + (a > 5.f);
+    if (TIES == 0) {                                       // (a search: the seven compares and adds bounded the quantizer)
+        const bool h = a > 1.75f, m = a > (h ? 3.5f : .75f);
+        const bool l = a > (h ? (m ? 5.f : 2.5f) : (m ? 1.25f : .25f));
+        return (h ? 4u : 0u) + (m ? 2u : 0u) + (l ? 1u : 0u);
+    }
     return (a > .25f) + (a >= .75f) + (a > 1.25f) + (a >= 1.75f) + (a > 2.5f) + (a >= 3.5f) + (a > 5.f);
 }
 
@@ -48,11 +51,15 @@ __device__ __forceinline__ float e2m1_val(uint32_t c) {
     return (c & 8) ? -v : v;
 }
 
-// floor / ceil of log2 of a positive normal fp32 value, from its exponent bits.
+// floor of log2 of a positive normal fp32 value, from its exponent bits.
 __device__ __forceinline__ int ilog2_floor(float v) { return (int)((__float_as_uint(v) >> 23) & 0xff) - 127; }
-__device__ __forceinline__ int ilog2_ceil(float v) {
-    const uint32_t u = __float_as_uint(v);
-    return (int)((u >> 23) & 0xff) - 127 + ((u & 0x7fffffu) != 0);
+
+// min(127, max(-127, ceil(log2(RN(max(amax, 1e-30) / 6))))) without the division: for amax = m 2^E, 1 <= m < 2, the quotient
+// is (m / 1.5) 2^(E - 2), so the value is E - 2 for m <= 1.5 (a quotient that rounds up to 2^(E - 2) included) and E - 1 beyond
+// (the next m above 1.5 gives 1 + 2/3 ulp, which rounds to 1 + ulp); infinity clamps to 127.
+__device__ __forceinline__ int e2m1_exp(float amax) {
+    const uint32_t u = __float_as_uint(fmaxf(amax, 1e-30f));
+    return u >= 0x7f800000u ? 127 : (int)((u + 0x3fffffu) >> 23) - 129;
 }
 
 // ------------------------------------------------------------------------------------------------ weight pack
@@ -79,7 +86,7 @@ __global__ __launch_bounds__(64) void mx_pack_kernel(const float* __restrict__ w
     if (MODE == 2) {
         e = ilog2_floor(fmaxf(amax, 1e-30f)) - 2;
     } else {
-        e = min(127, max(-127, ilog2_ceil(div_rn(fmaxf(amax, 1e-30f), 6.0f))));
+        e = e2m1_exp(amax);
         if (MODE == 1) {
             // the power of two among e and e - 1 with the smaller squared error, summed as numpy sums 32 float32
             // values (eight strided partial sums, then a fixed tree)
@@ -144,20 +151,20 @@ __host__ __device__ __forceinline__ int64_t mx_act_panel_offset(int64_t row, int
 // sign bit set for every negative input.  AF 0: tests/quant_sim.py:75-81 (mxfp8): e = floor(log2(max(amax, 1e-30))) - 8,
 // codes e4m3(clamp(x / 2^e, +-448)) nearest even.  XF32: fp32 input, else bf16.  Rows >= n_rows are skipped.
 // PAN (e4m3 only): q in the panel layout mx_act_panel_offset defines instead of row-major.
-// Memory bounds it.  A thread per block read 64 bytes on its own, one 64-byte line per lane and load, and left a panel
+// Memory bounds it (the e2m1 codes' compares beyond 4096 x 13824: 8192 x 17408 bf16 100 -> 86 us with the search in e2m1_mag and
+// no division in e2m1_exp, which four lanes now do where one did).  A thread per block read 64 bytes on its own, one 64-byte line per lane and load, and left a panel
 // chunk's stores to sixteen workgroups; here a wave's loads are contiguous (1 KB of bf16), and a panel workgroup owns
 // whole 2 KB chunks: 16 rows x 128 inputs, four of them requested at once.
-template <int AF, bool XF32, bool PAN = false>
+template <int AF, bool XF32, bool PAN = false, int U = PAN ? 4 : 1>       // U: 8-input pieces per thread
 __global__ __launch_bounds__(256) void mx_quant_act_kernel(const void* __restrict__ x, int64_t ldx,
                                                            const float* __restrict__ inv, uint8_t* __restrict__ q,
                                                            uint8_t* __restrict__ s,
                                                            const int32_t* __restrict__ n_rows, int M, int K) {
-    constexpr int U = PAN ? 4 : 1;                         // 8-input pieces per thread
     const int tid = threadIdx.x;
     const int row = PAN ? blockIdx.y * 16 + (tid >> 4) : blockIdx.y;
     int k[U];                                              // piece u: inputs k[u] .. + 7 (whole 32-input blocks in range)
 #pragma unroll
-    for (int u = 0; u < U; u++) k[u] = PAN ? (blockIdx.x * U + u) * 128 + (tid & 15) * 8 : (blockIdx.x * 256 + tid) * 8;
+    for (int u = 0; u < U; u++) k[u] = PAN ? (blockIdx.x * U + u) * 128 + (tid & 15) * 8 : ((blockIdx.x * U + u) * 256 + tid) * 8;
     float v[U][8];
     const int64_t lrow = min(row, M - 1);                  // loads first, in range; the row count is read under them
 #pragma unroll
@@ -210,7 +217,7 @@ __global__ __launch_bounds__(256) void mx_quant_act_kernel(const void* __restric
             uint8_t* d = PAN ? q + mx_act_panel_offset(row, k[u], K) : q + (int64_t)row * K + k[u];
             *reinterpret_cast<v2u*>(d) = v2u{w[0], w[1]};
         } else {
-            e = min(127, max(-127, ilog2_ceil(div_rn(fmaxf(amax, 1e-30f), 6.0f))));
+            e = e2m1_exp(amax);
             const float r = pow2i(-e);
             uint32_t w = 0;
 #pragma unroll
@@ -1143,6 +1150,9 @@ extern "C" int prism_mxfp4_quant_act(const void* x, int x_f32, int64_t ldx, cons
         else hipLaunchKernelGGL((mx_quant_act_kernel<0, false, true>), grid, dim3(256), 0, st, x, ldx, inv, q, s,
                                 n_rows, (int)M, (int)K);
     } else if (fmt == PRISM_MX_E4M3) { if (x_f32) QA(0, true); else QA(0, false); }
+    else if (!x_f32 && M > 1024 && K > 16384)              // long batches of long rows: two loads in flight (8192 x 17408 80
+        hipLaunchKernelGGL((mx_quant_act_kernel<4, false, false, 2>), dim3((unsigned)((K + 4095) / 4096), (unsigned)M),
+                           dim3(256), 0, st, x, ldx, inv, q, s, n_rows, (int)M, (int)K);           // against 86 us)
     else { if (x_f32) QA(4, true); else QA(4, false); }
 #undef QA
     PRISM_LAUNCH_CHECK();
