@@ -217,11 +217,12 @@ PRISM_API int prism_q4k_pack(const uint8_t* raw, uint8_t* qv, uint8_t* meta, int
  *   epi 0: bf16(y); epi 1: out = RN(out + y).
  * xq int8 [M, K]; a fp32, element (b, m) at a[b * a_sb + m] (a_sb = 0: one scale per token); xs int8 [K/256, M, 16]
  * (per super-block eight S & 63 then eight S >> 6); qv / meta from prism_q4k_pack; out row stride ldo.
- * kernel: -1 picks by shape (2 up to 4 rows where it applies and N / 16 < 512, else 1 up to 16 rows; beyond 16 rows the
- * split-round kernel of w4a8_mid.hip where few 128 x 128 tiles would leave CUs idle, else 0); 0 the prefill tile kernel;
+ * kernel: -1 picks by shape (2 up to 4 rows where it applies and N / 16 < 512, else 1 up to 16 rows; beyond 16 rows 4
+ * where few 128 x 128 tiles would leave CUs idle, else 0); 0 the prefill tile kernel;
  * 1 the per-tile decode kernel (M <= 16; the tile kernel when its per-super-block terms, K/256 x M x 64 bytes, exceed
  * the 160 KB of LDS); 2 the balanced-grid decode kernel (M <= 16 with M (K + 32) + K M / 8 bytes of activation image
- * within LDS; equal shares of the weights per CU, running sums handed between workgroups through `workspace`).
+ * within LDS; equal shares of the weights per CU, running sums handed between workgroups through `workspace`); 4 the mid
+ * kernel, for batches whose 128 x 128 tiles leave CUs idle (M <= 4096, K <= 2^23).
  * workspace: for kernel 2, a zero-initialised device buffer of at least prism_w8a8_q8_0_packed_workspace_bytes(N, K)
  * bytes (the same size rule as the Q8_0 one), left zeroed by every call; may be null for the other kernels.  Calls
  * sharing one workspace must not overlap in time.  Needs K % 256 == 0, N % 16 == 0.
@@ -356,9 +357,9 @@ PRISM_API int prism_mxfp4_quant_act(const void* x, int x_f32, int64_t ldx, const
  * prism_mxfp4_pack / _repack.  epi 0: bf16 out; epi 1: out (fp32) = out + y.  Output row stride ldo.  n_rows may be
  * null (all M rows live).  Every kernel sums in the same order (128-input MFMA steps chained within 1024-input
  * segments, segment sums added left to right), so results do not depend on M or on the kernel.
- * kernel: -1 picks by shape, one more kernel among them for batches whose tiles leave CUs idle; 0 the tile kernel; 1 the
- * decode kernel (M <= 64); 2 the split decode, which needs the
- * workspace of prism_mxfp4_gemm_ws (here: PRISM_ERR_ARG).  Needs N % 16 == 0, K % 128 == 0.
+ * kernel: -1 picks by shape, 0 the tile kernel; 1 the decode kernel (M <= 64); 2 the split decode, which needs the
+ * workspace of prism_mxfp4_gemm_ws (here: PRISM_ERR_ARG); 3 the mid kernel, for batches whose tiles leave CUs idle
+ * (row-major activations, M <= 65536, K <= 2^22, as 4-byte aligned).  Needs N % 16 == 0, K % 128 == 0.
  * a_fmt PRISM_MX_E4M3_PANELS (activations from prism_mxfp4_quant_act in that format): the tile kernel only (kernel
  * -1 or 0; N K / 2 < 2^31), bits equal to the row-major e4m3 call's.
  */

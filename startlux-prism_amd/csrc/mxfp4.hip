@@ -1043,10 +1043,11 @@ static void mx_mid_go(int nw, const uint8_t* aq, const uint8_t* as, const uint8_
 // 16-row activation tiles per workgroup: up to four of e2m1 rows, three of e4m3 (four spill registers: 64 x 13824 x 5120
 // 47 us), in equal row groups.
 struct MxMidRows {
+    static constexpr int most(int a_fmt) { return a_fmt == PRISM_MX_E2M1 ? 4 : 3; }
     int gy, mt;
     MxMidRows(int a_fmt, int64_t M) {
-        const int64_t t = (M + 15) / 16, most = a_fmt == PRISM_MX_E2M1 ? 4 : 3;
-        gy = (int)((t + most - 1) / most);
+        const int64_t t = (M + 15) / 16;
+        gy = (int)((t + most(a_fmt) - 1) / most(a_fmt));
         mt = (int)((t + gy - 1) / gy);
     }
 };
@@ -1056,11 +1057,12 @@ struct MxMidRows {
 template <int AF>
 static void mx_mid_launch(const uint8_t* aq, const uint8_t* as, const uint8_t* wq, const uint8_t* ws, void* out,
                           int64_t ldo, const int32_t* n_rows, int M, int N, int K, int epi, hipStream_t st) {
+    static_assert(PRISM_MX_E4M3 == 0 && PRISM_MX_E2M1 == 4, "AF is the format");
     const MxMidRows rows(AF, M);
     const int gy = rows.gy, mt = rows.mt;
     const int nseg = (K / kMxStep + kMxSegSteps - 1) / kMxSegSteps, rounds = (nseg + kMxMidWaves - 1) / kMxMidWaves;
     const int nw = (nseg + rounds - 1) / rounds;           // equal rounds
-    constexpr int M4 = AF == 0 ? 3 : 4;
+    constexpr int M4 = MxMidRows::most(AF);
 #define MXM(TGV, MTV)                                                                                                \
     do {                                                                                                             \
         if (epi) mx_mid_go<AF, TGV, MTV, 1>(nw, aq, as, wq, ws, out, ldo, n_rows, M, N, K, gy, st);                  \
@@ -1076,7 +1078,12 @@ static void mx_mid_launch(const uint8_t* aq, const uint8_t* as, const uint8_t* w
 #undef MXM
 }
 
-// Whether the mid kernel takes the shape.  Up to 16 rows: e2m1 batches from 20 M weights (16 x 34816 x 5120 30.1 -> 21.7 us,
+// 32-bit offsets inside a workgroup's operands; activations by rows.
+static bool mx_mid_fits(int a_fmt, int64_t M, int64_t K) {
+    return a_fmt != PRISM_MX_E4M3_PANELS && K <= (1 << 22) && M <= (1 << 16);
+}
+
+// Whether the mid kernel takes the shape by default.  Up to 16 rows: e2m1 batches from 20 M weights (16 x 34816 x 5120 30.1 -> 21.7 us,
 // 5120^2 at 1 / 16 rows 6.2 / 9.2 -> 5.6 / 6.8; 1 x 1024 x 5120 3.8 against 4.7), and of e4m3 the wide ones the split
 // decode would take (34816 x 5120 at 1 / 16 rows 26.3 / 25.9 -> 19.9 / 22.9 us; at 5120 x 17408 and 16 rows the split stays
 // ahead, 16.7 against 17.5).  Beyond, from 8 M weights (17 x 1024 x 2048 4.1 against 4.6), measured at K = 5120 (both sides go with K): about 3 us and
@@ -1084,7 +1091,7 @@ static void mx_mid_launch(const uint8_t* aq, const uint8_t* as, const uint8_t* w
 // one per CU, 45 us per round of two beyond (us, mid / tile: e2m1 24 x 34816 28.1 / 27.9, 64 x 13824 21 / 29, 128 x 5120
 // 19.1 / 20.3, 128 x 13824 37 / 28; e4m3 32 x 13824 16 / 27.5, 40 x 5120 10.5 / 22).
 static bool mx_mid_faster(int a_fmt, int64_t M, int64_t N, int64_t K, bool split) {
-    if (a_fmt == PRISM_MX_E4M3_PANELS || K > (1 << 22) || M > (1 << 16)) return false;    // 32-bit offsets
+    if (!mx_mid_fits(a_fmt, M, K)) return false;
     if (M <= 16) return a_fmt == PRISM_MX_E2M1 ? N * K >= (20LL << 20) : split && N > 8192;
     if (N * K < (8LL << 20)) return false;
     const MxMidRows rows(a_fmt, M);
@@ -1174,7 +1181,7 @@ extern "C" int prism_mxfp4_gemm_ws(const uint8_t* aq, const uint8_t* as, int a_f
     hipStream_t st = (hipStream_t)stream;
     const int MT = (int)((M + 15) / 16);
     if (a_fmt == PRISM_MX_E4M3_PANELS) {                 // the direct-weight tile kernel only
-        if (kernel == 1 || kernel == 2 || (int64_t)N * K / 2 >= (1LL << 31)) return PRISM_ERR_SHAPE;
+        if (kernel == 1 || kernel == 2 || kernel == 3 || (int64_t)N * K / 2 >= (1LL << 31)) return PRISM_ERR_SHAPE;
         kernel = 0;
     }
     // the split decode: one 16-row block of e4m3 rows, its workspace, ranges of at most T units (two segments)
@@ -1186,7 +1193,10 @@ extern "C" int prism_mxfp4_gemm_ws(const uint8_t* aq, const uint8_t* as, int a_f
     // measured against the staged decode at 1-16 rows: 15.8-16.0 against 17.3-18.8 us at 17408 x 5120, 16.9
     // against 18.2-20.6 at 5120 x 17408, 21.5-21.7 against 23.5-25.6 at 27648 x 5120; slower below about 80 M weights
     // (its second launch costs about 2.5 us: 8.5 against 6.7-7.3 us at 5120^2, 14.0 against 11.4 at 8192^2)
-    if (kernel < 0 && PRISM_ALIGNED(as, 4) && mx_mid_faster(a_fmt, M, N, K, split_ok && N * K >= (80LL << 20))) {
+    if (kernel == 3 && !mx_mid_fits(a_fmt, M, K)) return PRISM_ERR_SHAPE;
+    if (kernel == 3 && !PRISM_ALIGNED(as, 4)) return PRISM_ERR_ALIGN;
+    if (kernel < 0 && PRISM_ALIGNED(as, 4) && mx_mid_faster(a_fmt, M, N, K, split_ok && N * K >= (80LL << 20))) kernel = 3;
+    if (kernel == 3) {
         if (a_fmt == PRISM_MX_E4M3) mx_mid_launch<0>(aq, as, wq, ws, out, ldo, n_rows, (int)M, (int)N, (int)K, epi, st);
         else mx_mid_launch<4>(aq, as, wq, ws, out, ldo, n_rows, (int)M, (int)N, (int)K, epi, st);
         PRISM_LAUNCH_CHECK();

@@ -866,16 +866,17 @@ extern "C" int prism_w4a8_q4k_gemm(const int8_t* xq, const float* a, int64_t a_s
         return PRISM_ERR_SHAPE;
     if (!PRISM_ALIGNED(xq, 16) || !PRISM_ALIGNED(xs, 16) || !PRISM_ALIGNED(qv, 16) || !PRISM_ALIGNED(meta, 16))
         return PRISM_ERR_ALIGN;
-    if (kernel < -1 || kernel > 2) return PRISM_ERR_ARG;
+    if (kernel < -1 || kernel > 4 || kernel == 3) return PRISM_ERR_ARG;
+    if (kernel == 4 && !w4_mid_fits(M, K)) return PRISM_ERR_SHAPE;
     const bool can_bal = q4k_bal_fits(M, N, K) && workspace && workspace_bytes >= q4k_bal_workspace_bytes(N);
     // by default up to 4 rows: the balanced kernel for long projections of fewer than two 16-row tiles per CU (where
     // a tile per workgroup leaves CUs with one tile more than others: 5120 x 17408 at 1 row 15.1 us against 18.4 us),
     // given its workspace; the per-tile kernel otherwise (13824 x 5120: 11.4 against 15.4 us; 5120^2 at 1-4 rows
     // 7.5-8.0 against 8.2-8.8 us) and from 5 rows, where it takes two tiles per workgroup (5120^2 at 16 rows 8.9
-    // against 9.9 us); beyond 16 rows the mid kernel (3, w4a8_mid.hip) where it is the faster one, else the tile kernel.  The
-    // MI355X table overrides this per shape up to 16 rows.
+    // against 9.9 us); beyond 16 rows the mid kernel (w4a8_mid.hip) where it is the faster one, else the tile kernel.  The
+    // MI355X table overrides this per shape.
     if (kernel == -1) kernel = M >= 1 && M <= 16 ? (can_bal && N / 16 < 512 && K >= 8192 && M <= 4 ? 2 : 1) :
-                                 w4_mid_faster(false, M, N, K) ? 3 : 0;
+                                 w4_mid_faster(false, M, N, K) ? 4 : 0;
     if (kernel == 1 && M > 16) return PRISM_ERR_ARG;
     if (kernel == 2 && !can_bal) return M > 16 || !q4k_bal_fits(M, N, K) ? PRISM_ERR_SHAPE : PRISM_ERR_ARG;
     if (M == 0) return PRISM_OK;
@@ -911,7 +912,7 @@ extern "C" int prism_w4a8_q4k_gemm(const int8_t* xq, const float* a, int64_t a_s
         else { if (epi == 0) W4S_TG(4, 0); else W4S_TG(4, 1); }
 #undef W4S_TG
 #undef W4S
-    } else if (kernel == 3) {
+    } else if (kernel == 4) {
         w4_mid_launch(xq, a, a_sb, xs, qv, meta, out, ldo, n_rows, Mi, Ni, Ki, epi, st);
     } else if ((int64_t)(N / 16) * (K / 256) * 2048 < ((int64_t)1 << 31) && M * K < ((int64_t)1 << 31)) {
         // the 128 x 128 tile kernel (w4a8_prefill.hip), whose stage offsets are 32-bit
@@ -949,8 +950,9 @@ extern "C" int prism_w4a8_q6k_gemm(const int8_t* xq, const float* a, int64_t a_s
     if (M < 0 || N <= 0 || K <= 0 || N % 16 || K % 256 || ldo < N || M > (1 << 30) || N > (1 << 30) || K > (1 << 30))
         return PRISM_ERR_SHAPE;
     if (!PRISM_ALIGNED(xq, 16) || !PRISM_ALIGNED(qv, 16) || !PRISM_ALIGNED(meta, 16)) return PRISM_ERR_ALIGN;
-    if (kernel < -1 || kernel > 2) return PRISM_ERR_ARG;
-    if (kernel == -1) kernel = M <= 16 ? 1 : w4_mid_faster(true, M, N, K) ? 3 : 0;
+    if (kernel < -1 || kernel > 4 || kernel == 3) return PRISM_ERR_ARG;
+    if (kernel == 4 && !w4_mid_fits(M, K)) return PRISM_ERR_SHAPE;
+    if (kernel == -1) kernel = M <= 16 ? 1 : w4_mid_faster(true, M, N, K) ? 4 : 0;
     if ((kernel == 1 || kernel == 2) && M > 16) return PRISM_ERR_ARG;
     if (M == 0) return PRISM_OK;
     hipStream_t st = (hipStream_t)stream;
@@ -996,7 +998,7 @@ extern "C" int prism_w4a8_q6k_gemm(const int8_t* xq, const float* a, int64_t a_s
         }
 #undef Q6DEC_
 #undef Q6DEC
-    } else if (kernel == 3) {
+    } else if (kernel == 4) {
         w4_mid_launch(xq, a, a_sb, nullptr, qv, meta, out, ldo, n_rows, Mi, Ni, Ki, epi, st);
     } else if ((int64_t)(N / 16) * (K / 256) * 4096 < ((int64_t)1 << 31) && M * K < ((int64_t)1 << 31)) {
         // the 128 x 128 two-plane tile kernel (w4a8_prefill.hip), whose stage offsets are 32-bit

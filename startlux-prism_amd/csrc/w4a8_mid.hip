@@ -279,8 +279,9 @@ template <bool Q6, int NW, int TG>
 static void mid_mt(int mt, int epi, const int8_t* xq, const float* a, int64_t a_sb, const int8_t* xs,
                    const uint8_t* qv, const uint8_t* meta, void* out, int64_t ldo, const int32_t* n_rows, int M, int N,
                    int K, int gy, hipStream_t st) {
-    // (two tiles, four row tiles: the Q4_K form of four waves only)
+    // (two tiles, four row tiles: the Q4_K form of four waves only; the others would take the rows in more groups)
     constexpr int M4 = TG == 2 && (Q6 || NW == 8) ? 3 : 4;
+    if (mt > M4) gy = ((M + 15) / 16 + M4 - 1) / M4;
     if (mt <= 2) epi == 0 ? mid_go<Q6, NW, TG, 2, 0>(MID_ARGS) : mid_go<Q6, NW, TG, 2, 1>(MID_ARGS);
     else if (mt == 3) epi == 0 ? mid_go<Q6, NW, TG, 3, 0>(MID_ARGS) : mid_go<Q6, NW, TG, 3, 1>(MID_ARGS);
     else epi == 0 ? mid_go<Q6, NW, TG, M4, 0>(MID_ARGS) : mid_go<Q6, NW, TG, M4, 1>(MID_ARGS);
@@ -310,7 +311,7 @@ void w4_mid_launch(const int8_t* xq, const float* a, int64_t a_sb, const int8_t*
 // outputs, the tile kernel 45 us for each round of one 128 x 128 tile per CU, whatever the rows in it: 64 x 13824 30
 // against 45 us, 100 x 13824 51 against 47, 128 x 5120 25 against 44.
 bool w4_mid_faster(bool q6k, int64_t M, int64_t N, int64_t K) {
-    if (M > 4096 || K > (1 << 23)) return false;       // 32-bit offsets inside a workgroup's operands
+    if (!w4_mid_fits(M, K)) return false;
     const int64_t blocks = (M + 15) / 16 * (N / 16), tiles = (M + 127) / 128 * ((N + 127) / 128);
     return 30000 + (q6k ? 100 : 87) * blocks < (tiles + 255) / 256 * 450000;
 }

@@ -24,7 +24,7 @@ from . import scratch
 QK = 32
 E4M3, E4M3_PANELS, E2M1 = 0, 1, 4
 MODES = {"max": 0, "mse": 1, "ocp": 2}
-KERNELS = {"auto": -1, "tile": 0, "decode": 1, "split": 2}
+KERNELS = {"auto": -1, "tile": 0, "decode": 1, "split": 2, "mid": 3}
 SPLIT_WS_BYTES = 32 << 20     # the split decode's segment sums: 1 KB per (1024-input segment, 16-row tile)
 _WS = scratch.Scratch(SPLIT_WS_BYTES)
 

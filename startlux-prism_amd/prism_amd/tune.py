@@ -6,8 +6,8 @@ bench/cuda_gemm_micro.py --table and bench/w4a8_table.py.
 For each projection shape of the 27B model (the shapes of the reference's tables, kernels/gemm_table_h200.json and
 w4a8_table_h200.json, with N a multiple of 16) and each of the reference's token buckets, every kernel valid at that
 token count is timed with its weights streamed from HBM (copies rotated through more than 3 x the 256 MB MALL, the
-launches replayed from a HIP graph) and the fastest is recorded.  W4A8 beyond 16 rows is left to the library's own
-rule.  Every kernel computes the same bits, so the table changes speed only.
+launches replayed from a HIP graph) and the fastest is recorded.  (The committed W4A8 table ends at 16 rows: beyond them the
+library's own rule picks between the same kernels.)  Every kernel computes the same bits, so the table changes speed only.
 """
 import argparse
 import json
@@ -129,13 +129,14 @@ def tune_w4(shapes, Ms, dev, log):
         nbytes = base.qv.numel() + base.meta.numel()
         ws = [base] + [KW4.W4(kind, base.qv.clone(), base.meta.clone(), N, K) for _ in range(_copies(nbytes) - 1)]
         row = {}
-        for M in (m for m in Ms if m <= 16):
+        for M in Ms:
             xq = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8, device=dev)
             a = torch.rand(1, M, generator=g, device=dev)
             xs = torch.randint(-64, 64, (K // 256, M, 16), generator=g, dtype=torch.int8, device=dev)
             out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
             n = torch.tensor([M], dtype=torch.int32, device=dev)
-            best, us = _pick(["decode", "stream", "tile"], lambda c: (lambda i: KW4.gemm(xq, a, xs, ws[i], out, n, kernel=c)), len(ws), M)
+            cands = ["decode", "stream", "mid", "tile"] if M <= 16 else ["mid", "tile"] if M <= 4096 else ["tile"]
+            best, us = _pick(cands, lambda c: (lambda i: KW4.gemm(xq, a, xs, ws[i], out, n, kernel=c)), len(ws), M)
             row[str(M)] = [best]
             if us:
                 log(f"{kind} {N}x{K} M={M}: " + " ".join(f"{c} {t:.1f}" for c, t in us.items()) + f" -> {best}")

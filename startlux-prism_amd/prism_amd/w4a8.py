@@ -28,7 +28,7 @@ from .gguf_formats import KQuant, Q4_K_BYTES, Q6_K_BYTES, kquant_kind
 QK_K = 256
 # "stream": on Q6_K the per-tile stream kernel, on Q4_K the balanced-grid kernel (up to 16 rows, its activation image
 # within LDS, with the device workspace of w8a8.workspace)
-KERNELS = {"auto": -1, "tile": 0, "decode": 1, "stream": 2}
+KERNELS = {"auto": -1, "tile": 0, "decode": 1, "stream": 2, "mid": 4}
 
 
 class W4(NamedTuple):
@@ -175,7 +175,7 @@ def gemm(xq, a, xs, w: W4, out, n_rows, epi=0, cfg=None, pdl=0, kernel="auto"):
         raise ValueError(f"out must be {want} [>= {M}, >= {w.n}] with unit column stride")
     if kernel == "auto":             # the MI355X table's choice for the shape, where valid (dispatch.w4a8_kernel); its
         c = dispatch.w4a8_kernel(w.kind, w.n, K, M)      # entries end at 16 rows, beyond which the library's rule picks
-        ok = c == "tile" or (c in ("decode", "stream") and M <= 16)
+        ok = c == "tile" or (c in ("decode", "stream") and M <= 16) or (c == "mid" and M <= 4096 and K <= 1 << 23)
         kernel = c if ok else "auto"
     if w.kind == "q6k":              # no mins: xs is not read
         L.call("prism_w4a8_q6k_gemm", L.ptr(xq), L.ptr(a), a_sb, L.ptr(w.qv), L.ptr(w.meta), L.ptr(out),

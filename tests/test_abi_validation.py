@@ -66,7 +66,14 @@ def test_w4a8_q4k_gemm_checks(lib):
     assert call(kernel=2, M=17, ws=P, ws_bytes=1 << 20) == SHAPE     # at most 16 rows
     assert call(kernel=2, K=1 << 16, ws=P, ws_bytes=1 << 20) == SHAPE  # the activation image exceeds LDS
     assert call(kernel=1, M=17) == ARG
+    assert call(kernel=5) == ARG
+    assert call(kernel=4, M=4097) == SHAPE       # the mid kernel's 32-bit offsets
+    assert call(kernel=4, K=(1 << 23) + 256) == SHAPE
+    assert call(kernel=4, M=0) == OK
     assert call(M=0) == OK
+    q6 = lib.prism_w4a8_q6k_gemm
+    assert [q6(P, P, 0, P, P, P, 64, P, M, 64, 512, 0, k, None) for k, M in ((3, 16), (5, 16), (4, 4097), (4, 0))] == \
+        [ARG, ARG, SHAPE, OK]
 
 
 def test_mxfp4_gemm_checks(lib):
@@ -78,6 +85,9 @@ def test_mxfp4_gemm_checks(lib):
     assert call(fmt=2) == ARG                    # neither e4m3 (0), e4m3 panels (1) nor e2m1 (4)
     assert call(fmt=1, kernel=1) == SHAPE        # panel activations: the tile kernel only
     assert call(fmt=1, M=0) == OK
+    assert call(fmt=1, kernel=3) == SHAPE
+    assert call(kernel=3, M=65537) == SHAPE      # the mid kernel's 32-bit offsets
+    assert call(kernel=3, K=(1 << 22) + 128) == SHAPE
     assert call(K=192) == SHAPE                  # K % 128
     assert call(aq=U) == ALIGN
     assert call(epi=1, out=P + 8) == ALIGN       # the fp32 residual needs 16-byte rows

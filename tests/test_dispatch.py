@@ -62,7 +62,7 @@ def test_off(tables, monkeypatch):
 
 LIMITS = {"gemm_table": {"decode": 1 << 20, "split": 512, "tile": 1 << 30}, "q8_table": {"decode": 64, "stream": 16, "mid": 1 << 20,
                                                                                    "tile": 1 << 30},
-          "w4a8_table": {"decode": 16, "stream": 16, "tile": 1 << 30}}
+          "w4a8_table": {"decode": 16, "stream": 16, "mid": 4096, "tile": 1 << 30}}
 
 
 @pytest.mark.parametrize("path", sorted(glob.glob(os.path.join(dispatch.HERE, "*_table_*.json"))))

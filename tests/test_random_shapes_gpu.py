@@ -82,13 +82,14 @@ def test_w8a8_per_channel_random(dev, case):
     _check(out, want, live, epi)
 
 
-@pytest.mark.parametrize("case", range(10))
+@pytest.mark.parametrize("case", range(14))
 def test_w4a8_q4k_random(dev, case):
     from prism_amd import gguf_formats as GF
     from prism_amd import w4a8 as KW4
     g = rng(3000 + case + BASE)
     M, live, N, K, epi = _draw(g, 256, 6144)
     kernel = str(g.choice(["tile"] + (["decode", "stream"] if M <= 16 else [])))
+    kernel = "mid" if case >= 10 else kernel
     group = int(g.choice([256, K]))
     blocks = O.q4k_quantize(weights_f32(N, K, seed=case + 7 + BASE))
     xq, a, xs = O.quant_rows_g(O.bf16_to_f32(acts_bf16(M, K, seed=case + 8 + BASE)), group)
@@ -102,13 +103,14 @@ def test_w4a8_q4k_random(dev, case):
     _check(out, want, live, epi)
 
 
-@pytest.mark.parametrize("case", range(10))
+@pytest.mark.parametrize("case", range(14))
 def test_w4a8_q6k_random(dev, case):
     from prism_amd import gguf_formats as GF
     from prism_amd import w4a8 as KW4
     g = rng(4000 + case + BASE)
     M, live, N, K, epi = _draw(g, 256, 6144)
     kernel = str(g.choice(["tile"] + (["decode", "stream"] if M <= 16 else [])))
+    kernel = "mid" if case >= 10 else kernel
     blocks = q6k_random_blocks(N, K // 256, seed=case + 9 + BASE)
     xq, a, _ = O.quant_rows_g(O.bf16_to_f32(acts_bf16(M, K, seed=case + 10 + BASE)), 256)
     base = g.standard_normal((M, N)).astype(np.float32)
@@ -121,12 +123,13 @@ def test_w4a8_q6k_random(dev, case):
     _check(out, want, live, epi)
 
 
-@pytest.mark.parametrize("case", range(8))
+@pytest.mark.parametrize("case", range(12))
 def test_mxfp4_random(dev, case):
     from prism_amd import mxfp4 as MX
     g = rng(5000 + case + BASE)
     M, live, N, K, _ = _draw(g, 128, 4096)
     kernel = str(g.choice(["tile"] + (["decode"] if M <= 64 else []) + (["split"] if M <= 16 else [])))
+    kernel = "mid" if case >= 8 else kernel
     w = weights_f32(N, K, seed=case + 11 + BASE)
     x = acts_bf16(M, K, seed=case + 12 + BASE)
     mw = MX.pack(_t(w, dev), "ocp")
