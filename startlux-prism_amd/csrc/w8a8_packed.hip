@@ -697,6 +697,9 @@ static void launch_packed(int kernel, const int8_t* a, const float* a_s, int64_t
             hipLaunchKernelGGL((w8a8_packed_mid_kernel<8, 1, 1, EPI>), dim3(N / 16, (M + 15) / 16), dim3(64), 0, st,
                                a, a_s, as_sm, qt, dt, out, ldo, n_rows, M, N, K);
     } else if (kernel == 0 || kernel == 3) {
+        int64_t cost = 0;
+        const int nt = kernel == 3 ? 4 : q8_tile_nt(M, N, &cost);
+        if (nt == 2) pan = nullptr;                  // (hardly a shape wide and long enough for panels takes 64 columns)
         if (pan)                                     // the panel copy first, then the tile kernel reads it
             hipLaunchKernelGGL(q8_act_panel_kernel, dim3((unsigned)((K + 511) / 512), (unsigned)((M + 127) / 128 * 4)),
                                dim3(256), 0, st, a, pan, M, K);
@@ -711,12 +714,14 @@ static void launch_packed(int kernel, const int8_t* a, const float* a_s, int64_t
         if (kernel == 3) {
             if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 4, true>), 128);
             else Q8T((w8a8_q8_tile_kernel<EPI, false, 4, true>), 128);
+        } else if (nt == 4) {
+            if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 4>), 128);
+            else Q8T((w8a8_q8_tile_kernel<EPI, false, 4>), 128);
+        } else if (nt == 3) {
+            if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 3>), 96);
+            else Q8T((w8a8_q8_tile_kernel<EPI, false, 3>), 96);
         } else {
-            int64_t cost = 0;
-            const int nt = q8_tile_nt(M, N, &cost);
-            if (nt == 4) { if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 4>), 128); else Q8T((w8a8_q8_tile_kernel<EPI, false, 4>), 128); }
-            else if (nt == 3) { if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 3>), 96); else Q8T((w8a8_q8_tile_kernel<EPI, false, 3>), 96); }
-            else { if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 2>), 64); else Q8T((w8a8_q8_tile_kernel<EPI, false, 2>), 64); }
+            Q8T((w8a8_q8_tile_kernel<EPI, false, 2>), 64);
         }
 #undef Q8T
     }

@@ -23,9 +23,10 @@ def _run(dev, a, s, qs, d, epi, live=None, out0=None):
 
 
 # two, three and four column subtiles per wave (the last two need several hundred tiles); one, two and more stages; rows
-# and columns that end inside a tile, a wave and a subtile; panel activations (M >= 1024, N >= 16384)
+# and columns that end inside a tile, a wave and a subtile; panel activations (M >= 1024, N >= 16384) with four and with
+# three subtiles
 @pytest.mark.parametrize("M,N,K,live", [(1, 16, 128, 1), (33, 80, 384, 32), (130, 208, 256, 129), (300, 13840, 256, 290),
-                                        (500, 16384, 128, 500), (1100, 16400, 256, 1030)])
+                                        (500, 16384, 128, 500), (1100, 16400, 256, 1030), (1024, 17424, 384, 1001)])
 def test_tile_bits(dev, M, N, K, live):
     a, s = int8_acts(M, K, seed=M + N)
     qs, d = q8_weights(N, K, seed=K + N)
