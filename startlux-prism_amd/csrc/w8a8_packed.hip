@@ -265,7 +265,7 @@ constexpr int PBM = 128;
 // Waves with no live row only stage the weights and keep the barriers.  PAN: `a` is the panel copy of
 // q8_act_panel_kernel, a fragment one 1 KB piece; otherwise it is 32 rows' 32 bytes.
 template <int EPI, bool PAN, int NT, bool RA = false>
-__global__ __launch_bounds__(256, 2) void w8a8_q8_tile_kernel(const int8_t* __restrict__ a,
+__global__ __launch_bounds__(256, 2) void w8a8_packed_tile_kernel(const int8_t* __restrict__ a,
                                                                 const float* __restrict__ a_s, int64_t as_sm,
                                                                 const int8_t* __restrict__ qt,
                                                                 const uint16_t* __restrict__ dt,
@@ -712,16 +712,16 @@ static void launch_packed(int kernel, const int8_t* a, const float* a_s, int64_t
                            n_rows, M, N, K, tiles_m, tiles_n);                                                     \
     } while (0)
         if (kernel == 3) {
-            if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 4, true>), 128);
-            else Q8T((w8a8_q8_tile_kernel<EPI, false, 4, true>), 128);
+            if (pan) Q8T((w8a8_packed_tile_kernel<EPI, true, 4, true>), 128);
+            else Q8T((w8a8_packed_tile_kernel<EPI, false, 4, true>), 128);
         } else if (nt == 4) {
-            if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 4>), 128);
-            else Q8T((w8a8_q8_tile_kernel<EPI, false, 4>), 128);
+            if (pan) Q8T((w8a8_packed_tile_kernel<EPI, true, 4>), 128);
+            else Q8T((w8a8_packed_tile_kernel<EPI, false, 4>), 128);
         } else if (nt == 3) {
-            if (pan) Q8T((w8a8_q8_tile_kernel<EPI, true, 3>), 96);
-            else Q8T((w8a8_q8_tile_kernel<EPI, false, 3>), 96);
+            if (pan) Q8T((w8a8_packed_tile_kernel<EPI, true, 3>), 96);
+            else Q8T((w8a8_packed_tile_kernel<EPI, false, 3>), 96);
         } else {
-            Q8T((w8a8_q8_tile_kernel<EPI, false, 2>), 64);
+            Q8T((w8a8_packed_tile_kernel<EPI, false, 2>), 64);
         }
 #undef Q8T
     }
