@@ -156,6 +156,12 @@ __device__ __forceinline__ v2u buf_load8(__amdgpu_buffer_rsrc_t r, uint32_t voff
     return __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
 }
 
+// The turn of activation pieces from load order to MFMA operand order through 1 KB of a wave's LDS, 16 rows of 64 bytes: four
+// neighbouring lanes load a row's pieces 0..3 (the memory pipeline merges neighbouring lanes only: in operand order, a row per
+// lane, it takes four times as long), and row r's piece c lies at slot c ^ lds_turn(r / 4), so that the lane groups of the
+// 16-byte reads (0-3, 12-15, 20-27 and the others of 32) lie on distinct banks.
+__device__ __forceinline__ int lds_turn(int r4) { return ((r4 ^ (r4 << 1)) & 2) | (r4 >> 1); }
+
 // Waits until at most N vector-memory operations of this wave are outstanding.  The compiler does not count LDS-DMA
 // writes as producers of later LDS reads, so every DMA stage is closed by an explicit wait (then a barrier).
 template <int N>

@@ -893,12 +893,9 @@ int64_t mx_split_workspace_bytes(int64_t N, int64_t K) {     // 1 KB of segment 
 // A workgroup owns TG adjacent 16-row weight tiles and MT 16-row activation tiles; its waves take the 1024-input segments
 // in turn (wave w segment r NW + w of round r), each for all TG x MT blocks, and leave the segment sums in LDS, where
 // after one barrier per round wave b adds block b's sums left to right.  The decode kernel it replaces here had one tile
-// per workgroup, so every weight byte cost MT activation bytes (e2m1), loaded a row per lane: the memory pipeline merges
-// neighbouring lanes only, so each piece was an access of its own.  Here four neighbouring lanes load a row's 64 bytes
-// and the wave turns them in LDS (piece c of row r at slot c ^ mx_turn(r / 4): the read's lane groups, 0-3, 12-15, 20-27
-// and the others of 32, then lie on distinct banks), and the TG tiles share them.  Both operands are requested four steps
-// ahead.  Same MFMA chain per segment and segment order: the same bits.
-__device__ __forceinline__ int mx_turn(int r4) { return ((r4 ^ (r4 << 1)) & 2) | (r4 >> 1); }
+// per workgroup, so every weight byte cost MT activation bytes (e2m1), loaded a row per lane, each piece an access of its
+// own.  Here four neighbouring lanes load a row's 64 bytes, the wave turns them in LDS (lds_turn), and the TG tiles share
+// them.  Both operands are requested four steps ahead.  Same MFMA chain per segment and segment order: the same bits.
 constexpr int kMxMidWaves = 8;
 
 template <int AF, int TG, int MT, int EPI>
@@ -929,10 +926,10 @@ __global__ __launch_bounds__(64 * kMxMidWaves, 2) void mx_mid_kernel(const uint8
     uint32_t av[MT], sv[MT];
 #pragma unroll
     for (int j = 0; j < MT; j++) {
-        av[j] = (uint32_t)(min(m0 + 16 * j + (lane >> 2), M - 1) - m0) * abytes + 16 * ((lane & 3) ^ mx_turn(lane >> 4));
+        av[j] = (uint32_t)(min(m0 + 16 * j + (lane >> 2), M - 1) - m0) * abytes + 16 * ((lane & 3) ^ lds_turn(lane >> 4));
         sv[j] = (uint32_t)(min(m0 + 16 * j + r, M - 1) - m0) * (K / 32);
     }
-    const int xrd = r * 64 + 16 * (p ^ mx_turn(r >> 2));
+    const int xrd = r * 64 + 16 * (p ^ lds_turn(r >> 2));
 
     v4i w[4][TG], x[4][MT][AP];
     uint32_t wsc[4][TG];

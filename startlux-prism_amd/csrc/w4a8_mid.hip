@@ -56,20 +56,16 @@ __global__ __launch_bounds__(NW * 64, 2) void w4_mid_kernel(const int8_t* __rest
     const auto wr = buf_rsrc(qv + (int64_t)nt0 * NB * WB);
     const auto mr = buf_rsrc(meta + (int64_t)nt0 * NB * MB);
     const auto xr = buf_rsrc(xq + (int64_t)m0 * K);
-    // Activations: four consecutive lanes load a row's 64 bytes of a pair (in the MFMA's own order, a row per lane, the
-    // memory pipeline takes four times as long: it merges neighbouring lanes only) and the wave turns them in LDS, row r's
-    // 16-byte piece c at slot c ^ xf(r / 4), which keeps the reads' lane groups (0-3, 12-15, 20-27 and the others of 32) off
-    // each other's banks.
-    auto xf = [](int r4) { return ((r4 ^ (r4 << 1)) & 2) | (r4 >> 1); };
+    // activations: four consecutive lanes load a row's 64 bytes of a pair, and the wave turns them in LDS (lds_turn)
     const auto sr = buf_rsrc(Q6 ? (const int8_t*)nullptr : xs + (int64_t)m0 * 16);
     uint32_t xv[MT], xsv[MT];
 #pragma unroll
     for (int j = 0; j < MT; j++) {
         xsv[j] = (min(m0 + 16 * j + lm, M - 1) - m0) * 16;
-        xv[j] = (uint32_t)(min(m0 + 16 * j + (lane >> 2), M - 1) - m0) * K + 16 * ((lane & 3) ^ xf(lane >> 4));
+        xv[j] = (uint32_t)(min(m0 + 16 * j + (lane >> 2), M - 1) - m0) * K + 16 * ((lane & 3) ^ lds_turn(lane >> 4));
     }
     int8_t* xw = reinterpret_cast<int8_t*>(al + BUFS * NW * MR) + wv * MT * 1024;
-    const int xrd = lm * 64 + 16 * (q ^ xf(lm >> 2));
+    const int xrd = lm * 64 + 16 * (q ^ lds_turn(lm >> 2));
     const uint32_t wv6 = (32 * (q & 1) + lm) * 16 + 8 * (q >> 1);
 
     auto load_w = [&](int b, MidW<Q6>* c) {            // past the end: the last super-block again
