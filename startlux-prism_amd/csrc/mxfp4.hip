@@ -1083,7 +1083,8 @@ static bool mx_mid_fits(int a_fmt, int64_t M, int64_t K) {
 // Whether the mid kernel takes the shape by default.  Up to 16 rows: e2m1 batches from 20 M weights (16 x 34816 x 5120 30.1 -> 21.7 us,
 // 5120^2 at 1 / 16 rows 6.2 / 9.2 -> 5.6 / 6.8; 1 x 1024 x 5120 3.8 against 4.7), and of e4m3 the wide ones the split
 // decode would take (34816 x 5120 at 1 / 16 rows 26.3 / 25.9 -> 19.9 / 22.9 us; at 5120 x 17408 and 16 rows the split stays
-// ahead, 16.7 against 17.5).  Beyond, from 8 M weights (17 x 1024 x 2048 4.1 against 4.6), measured at K = 5120 (both sides go with K): about 3 us and
+// ahead, 16.7 against 17.5); with the weights streamed from HBM, as a model's are (already in the caches, the decode
+// kernel is ahead at 1-4 rows: 5120^2 3.9 against 5.3).  Beyond, from 8 M weights (17 x 1024 x 2048 4.1 against 4.6), measured at K = 5120 (both sides go with K): about 3 us and
 // 5.6 ns (e2m1) or 7.2 ns (e4m3) per 16 x 16 outputs, against the tile kernel's 21 us and 75 ns per 64 x 256 tile up to
 // one per CU, 45 us per round of two beyond (us, mid / tile: e2m1 24 x 34816 28.1 / 27.9, 64 x 13824 21 / 29, 128 x 5120
 // 19.1 / 20.3, 128 x 13824 37 / 28; e4m3 32 x 13824 16 / 27.5, 40 x 5120 10.5 / 22).

@@ -639,8 +639,8 @@ static int q8_tile_nt(int64_t M, int64_t N, int64_t* cost) {
     return best;
 }
 
-// Whether the register-fold kernel beats the tile kernel beyond 16 rows: it takes 16 x 32 outputs per wave and 21.7 ns a
-// wave at K = 5120 once they fill the chip (128 x 5120: 25 against 43 us; 128 x 13824: 75 against 80; 128 x 27648: 148
+// Whether the register-fold kernel beats the tile kernel beyond 16 rows: it takes 21.7 ns per 16 x 32 outputs (one wave's
+// from 33 rows, two waves' of 16 x 16 below) at K = 5120 once they fill the chip (128 x 5120: 25 against 43 us; 128 x 13824: 75 against 80; 128 x 27648: 148
 // against 79; 32 x 34816 76 against 62; 300 x 1024: 17 against 43).  Over the dispatch table's 320 shapes and row counts the
 // choice costs 0.3% on average against the faster of the two.
 static bool q8_mid_faster(int64_t M, int64_t N) {
