@@ -38,13 +38,16 @@ class Scratch:
         self._eager = {}                 # (device index, stream) -> buffer, in the order made
         self._captured = {}              # device index -> the zeroed bytes for captured calls, or None
 
-    def get(self, dev, zeroed=True):
-        """The buffer for a call on dev's current stream; zeroed: the call uses the zeroed bytes (and no others)."""
+    def get(self, dev, zeroed=True, need=None):
+        """The buffer for a call on dev's current stream; zeroed: the call uses the zeroed bytes (and no others); need: the
+        bytes the call has a use for, where they are known (all a captured one gets: a graph's pool keeps them)."""
         idx = dev.index if dev.index is not None else torch.cuda.current_device()
         if torch.cuda.is_current_stream_capturing():
             if idx not in self._captured:
                 return None
-            return self._captured[idx] if zeroed and self.zeroed else self._empty(idx, self.nbytes)
+            if zeroed and self.zeroed:
+                return self._captured[idx]
+            return self._empty(idx, self.nbytes if need is None else min(need, self.nbytes))
         key = (idx, L.raw_stream(idx))
         buf = self._eager.get(key)
         return self._make(key) if buf is None else buf

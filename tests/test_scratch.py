@@ -48,6 +48,9 @@ def test_captured_calls_share_with_no_eager_one(gpu, zeroed):
     a, b = s.get(DEV), s.get(DEV, zeroed=False)
     assert len({t.data_ptr() for t in (eager, a, b)}) == 3
     assert b.numel() == 64 and a.numel() == (zeroed or 64) and not (zeroed and a.any())
+    assert s.get(DEV, zeroed=False, need=40).numel() == 40 and s.get(DEV, zeroed=False, need=400).numel() == 64
+    gpu["capturing"] = False
+    assert s.get(DEV, need=40).data_ptr() == eager.data_ptr()
 
 
 def test_bounded(gpu):
