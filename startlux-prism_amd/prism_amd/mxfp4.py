@@ -29,11 +29,11 @@ SPLIT_WS_BYTES = 32 << 20     # the split decode's segment sums: 1 KB per (1024-
 _WS = scratch.Scratch(SPLIT_WS_BYTES)
 
 
-def split_workspace(dev, need=None):
+def split_workspace(dev, need=None, stream=None):
     """The workspace of the split decode (kernel "split") on dev's current stream: its segment sums, rewritten by every
     launch.  None under graph capture on a device with no eager call yet: "auto" then picks another kernel and "split"
     raises.  need: the bytes a call uses, all that a captured one gets."""
-    return _WS.get(dev, need=need)
+    return _WS.get(dev, True, need, stream)
 
 
 class MX4(NamedTuple):
@@ -202,15 +202,15 @@ def gemm(a_q, a_s, w: MX4, out, n_rows, epi=0, out_stride=None, kernel="auto"):
     if epi == 0 and out.dtype != torch.bfloat16 or epi == 1 and out.dtype != torch.float32:
         raise ValueError("mxfp4.gemm: epi 0 writes bf16, epi 1 adds into fp32")
     ldo = out.stride(0) if out_stride is None else out_stride
-    ws = None
+    st, ws = L.stream_of(a_q), None
     if fmt == E4M3 and M <= 16 and kernel in ("auto", "split"):
-        ws = split_workspace(a_q.device, max(16, (K + 1023) // 1024 * (N // 16) * 1024))
+        ws = split_workspace(a_q.device, max(16, (K + 1023) // 1024 * (N // 16) * 1024), st)
     if kernel == "split" and ws is None:
         raise L.PrismError('kernel "split" needs the device workspace, made outside graph capture: run one eager call '
                            'first')
-    scratch.call(ws is not None, "prism_mxfp4_gemm_ws", L.ptr(a_q), L.ptr(a_s), fmt, L.ptr(w.q), L.ptr(w.s), L.ptr(out),
-                 ldo, L.ptr(live), M, N, K, epi, KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(),
-                 L.stream_of(a_q))
+    call = L.call if ws is None else scratch.locked_call   # the split decode and the kernel that adds its segment sums
+    call("prism_mxfp4_gemm_ws", L.ptr(a_q), L.ptr(a_s), fmt, L.ptr(w.q), L.ptr(w.s), L.ptr(out), ldo, L.ptr(live), M, N, K,
+         epi, KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(), st)
 
 
 def cutlass_enabled():

@@ -10,7 +10,7 @@ replayed graph's, would be read instead).
     be replayed at the same time.  On a device with no eager call yet there is none (None).
 
 Calls of several threads on one stream share its buffer: a call that launches more than one kernel on it holds a lock
-(call), so that its launches stay together.
+(locked_call), so that its launches stay together.
 """
 import threading
 
@@ -20,12 +20,11 @@ from . import _lib as L
 
 STREAMS = 8
 _LOCK = threading.Lock()
+_capturing = torch._C._cuda_isCurrentStreamCapturing      # (in the path of every decode-size call)
 
 
-def call(shares, name, *args):
-    """_lib.call; shares: its launches hand scratch from one to the next."""
-    if not shares:
-        return L.call(name, *args)
+def locked_call(name, *args):
+    """_lib.call of an entry point whose launches hand scratch from one to the next."""
     with _LOCK:
         return L.call(name, *args)
 
@@ -38,17 +37,17 @@ class Scratch:
         self._eager = {}                 # (device index, stream) -> buffer, in the order made
         self._captured = {}              # device index -> the zeroed bytes for captured calls, or None
 
-    def get(self, dev, zeroed=True, need=None):
-        """The buffer for a call on dev's current stream; zeroed: the call uses the zeroed bytes (and no others); need: the
+    def get(self, dev, zeroed=True, need=None, stream=None):
+        """The buffer for a call on dev's current stream (its handle, if the caller has it); zeroed: the call uses the zeroed bytes (and no others); need: the
         bytes the call has a use for, where they are known (all a captured one gets: a graph's pool keeps them)."""
         idx = dev.index if dev.index is not None else torch.cuda.current_device()
-        if torch.cuda.is_current_stream_capturing():
+        if _capturing():
             if idx not in self._captured:
                 return None
             if zeroed and self.zeroed:
                 return self._captured[idx]
             return self._empty(idx, self.nbytes if need is None else min(need, self.nbytes))
-        key = (idx, L.raw_stream(idx))
+        key = (idx, L.raw_stream(idx) if stream is None else stream)
         buf = self._eager.get(key)
         return self._make(key) if buf is None else buf
 

@@ -186,10 +186,10 @@ def gemm(xq, a, xs, w: W4, out, n_rows, epi=0, cfg=None, pdl=0, kernel="auto"):
     Mx = xs.shape[1]
     if Mx != M:
         raise ValueError("xs rows must equal xq rows")
-    ws = KW8.workspace(xq.device) if M <= 16 and kernel in ("auto", "stream") else None
+    st = L.stream_of(xq)
+    ws = KW8.workspace(xq.device, 0, st) if M <= 16 and kernel in ("auto", "stream") else None
     if kernel == "stream" and ws is None:
         raise L.PrismError('kernel "stream" needs the device workspace, made outside graph capture: run one eager '
                            'call first')
     L.call("prism_w4a8_q4k_gemm", L.ptr(xq), L.ptr(a), a_sb, L.ptr(xs), L.ptr(w.qv), L.ptr(w.meta), L.ptr(out),
-           out.stride(0), L.ptr(n_rows), M, w.n, K, epi, KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(),
-           L.stream_of(xq))
+           out.stride(0), L.ptr(n_rows), M, w.n, K, epi, KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(), st)

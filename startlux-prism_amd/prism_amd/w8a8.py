@@ -199,13 +199,13 @@ Q8_WS_BYTES = Q8_HANDOFF_BYTES + (96 << 20)
 _WS = scratch.Scratch(Q8_WS_BYTES, zeroed=Q8_HANDOFF_BYTES)
 
 
-def workspace(dev, panels=0):
+def workspace(dev, panels=0, stream=None):
     """The workspace of the packed Q8_0 GEMM on dev's current stream (the reference schema's `workspace`, allocated once
     per device as kernels/cuda_ext.py:138-143 does): the "stream" kernel's handoff words, zeroed once and left zeroed by
     every launch, then the prefill's panel copy of the activations.  Under graph capture the words alone, or, for a call
     that copies `panels` bytes of activations, the room for that alone, and None on a device with no eager call yet (the words' zero fill would be a graph
     node): "auto" then picks another kernel and "stream" raises.  See scratch.py for what calls may share."""
-    return _WS.get(dev, zeroed=not panels, need=Q8_HANDOFF_BYTES + panels)
+    return _WS.get(dev, not panels, Q8_HANDOFF_BYTES + panels, stream)
 
 
 def _gemm_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
@@ -223,16 +223,17 @@ def _gemm_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
         raise ValueError(f"out must be {want} [>= {M}, >= {w.n}] with unit column stride")
     pan = (M + 127) // 128 * 128 * K if M >= 1024 and w.n >= 16384 and kernel in ("auto", "tile", "reassoc") else 0
     pan = pan if Q8_HANDOFF_BYTES + pan <= Q8_WS_BYTES else 0
-    ws = workspace(a.device, pan) if (M <= 16 and kernel in ("auto", "decode", "stream")) or pan else None
+    st, ws = L.stream_of(a), None
+    if pan or (M <= 16 and kernel in ("auto", "decode", "stream")):
+        ws = workspace(a.device, pan, st)
     if kernel == "stream" and ws is None and asked == "auto":
         kernel = "auto"             # the table's pick needs the workspace; the library then picks without it
     if kernel == "stream" and ws is None:
         raise L.PrismError('kernel "stream" needs the device workspace, made outside graph capture: run one eager '
                            'call first')
-    # (two launches with the panels: the copy and the tile kernel that reads it)
-    scratch.call(pan, "prism_w8a8_q8_0_packed_gemm", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt), L.ptr(w.dt),
-                 L.ptr(out), out.stride(0), L.ptr(n_rows), M, w.n, K, epi, KERNELS[kernel], L.ptr(ws),
-                 0 if ws is None else ws.numel(), L.stream_of(a))
+    call = scratch.locked_call if pan else L.call          # with panels, the copy and the tile kernel that reads it
+    call("prism_w8a8_q8_0_packed_gemm", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt), L.ptr(w.dt), L.ptr(out),
+         out.stride(0), L.ptr(n_rows), M, w.n, K, epi, KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(), st)
     return None
 
 
@@ -241,12 +242,12 @@ PC_WS_BYTES = 96 << 20        # as the reference's workspace (kernels/cuda_ext.p
 _PCWS = scratch.Scratch(PC_WS_BYTES)
 
 
-def pc_workspace(dev, need=None):
+def pc_workspace(dev, need=None, stream=None):
     """The workspace of the per-channel GEMM on dev's current stream: the split decode's int32 slots (kernel "split") or
     the tile kernel's panel copy of the activations (wide projections from 1024 rows), rewritten by every launch.  None
     under graph capture on a device with no eager call yet: "auto" then picks another kernel and "split" raises.  need: the
     bytes a call can use, all that a captured one gets."""
-    return _PCWS.get(dev, need=need)
+    return _PCWS.get(dev, True, need, stream)
 
 
 _PC_KERNELS = {"auto": -1, "tile": 0, "decode": 1, "split": 2}
@@ -271,16 +272,19 @@ def _gemm_pc_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
     # (ceil(M / 16) 16 K bytes; the library takes it from 1024 rows on projections at least 16384 wide) where it fits
     use_ws = kernel == "split" or (kernel in ("auto", "tile") and
                                    (M <= 512 or (M + 15) // 16 * 16 * K <= PC_WS_BYTES))
-    slots = (12 * M * w.n + 255) // 256 * 256 if M <= 512 else 0
-    ws = pc_workspace(a.device, slots + (M + 15) // 16 * 16 * K) if use_ws else None
+    st, ws = L.stream_of(a), None
+    if use_ws:
+        slots = (12 * M * w.n + 255) // 256 * 256 if M <= 512 else 0
+        ws = pc_workspace(a.device, slots + (M + 15) // 16 * 16 * K, st)
     if kernel == "split" and ws is None and asked == "auto":
         kernel = "auto"             # the table's pick needs the workspace; the library then picks without it
     if kernel == "split" and ws is None:
         raise L.PrismError('kernel "split" needs the device workspace, made outside graph capture: run one eager '
                            'call first')
-    scratch.call(ws is not None, "prism_w8a8_pc_packed_gemm_ws", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt),
-                 L.ptr(w.ws), int(w.ws.dtype == torch.float16), L.ptr(out), out.stride(0), L.ptr(n_rows), M, w.n, K, epi,
-                 _PC_KERNELS[kernel], L.ptr(ws), 0 if ws is None else ws.numel(), L.stream_of(a))
+    call = L.call if ws is None else scratch.locked_call   # the kernel that fills the workspace, the one that reads it
+    call("prism_w8a8_pc_packed_gemm_ws", L.ptr(a), L.ptr(a_s), a_s.stride(0), L.ptr(w.qt), L.ptr(w.ws),
+         int(w.ws.dtype == torch.float16), L.ptr(out), out.stride(0), L.ptr(n_rows), M, w.n, K, epi, _PC_KERNELS[kernel],
+         L.ptr(ws), 0 if ws is None else ws.numel(), st)
     return None
 
 

@@ -17,7 +17,7 @@ class _Stream:
 def gpu(monkeypatch):
     state = {"stream": 1, "capturing": False}
     monkeypatch.setattr(L, "raw_stream", lambda idx: state["stream"])
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    monkeypatch.setattr(scratch, "_capturing", lambda: state["capturing"])
     monkeypatch.setattr(torch.cuda, "current_stream", lambda idx=None: _Stream())
     monkeypatch.setattr(scratch.Scratch, "_empty", staticmethod(lambda idx, n: torch.full((n,), 7, dtype=torch.uint8)))
     return state
