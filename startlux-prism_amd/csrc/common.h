@@ -132,12 +132,12 @@ __device__ __forceinline__ void dma1(const void* g, void* lds) {
 // SGPR) and the lane's fixed part in one VGPR, so a streaming loop computes no per-load addresses in VGPRs.  Streamed
 // that way the compiler has no address temporaries to place in registers still awaiting an earlier load (which makes
 // it wait for the previous requests before issuing the next ones).  Raw buffer (stride 0): the range check compares
-// voffset + soffset with the record count, here the largest, so it never clips a valid offset.
+// voffset with the record count minus soffset, here the largest count, so it never clips a valid offset.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
 }
 // The same with the record count set to `bytes` from the base: a load past it returns zeros instead of reading beyond
-// the caller's buffer (the check is per dword).
+// the caller's buffer (the check is per dword).  soffset has to stay within `bytes`: the difference wraps beyond.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc_n(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }

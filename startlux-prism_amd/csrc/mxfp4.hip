@@ -54,9 +54,9 @@ __device__ __forceinline__ float e2m1_val(uint32_t c) {
 // floor of log2 of a positive normal fp32 value, from its exponent bits.
 __device__ __forceinline__ int ilog2_floor(float v) { return (int)((__float_as_uint(v) >> 23) & 0xff) - 127; }
 
-// min(127, max(-127, ceil(log2(RN(max(amax, 1e-30) / 6))))) without the division: for amax = m 2^E, 1 <= m < 2, the quotient
-// is (m / 1.5) 2^(E - 2), so the value is E - 2 for m <= 1.5 (a quotient that rounds up to 2^(E - 2) included) and E - 1 beyond
-// (the next m above 1.5 gives 1 + 2/3 ulp, which rounds to 1 + ulp); infinity clamps to 127.
+// min(127, max(-127, ceil(log2(RN(max(amax, 1e-30) / 6))))) without the division: for amax = m 2^E, 1 <= m < 2, the
+// quotient is (m / 1.5) 2^(E - 2), so the value is E - 2 for m <= 1.5 (a quotient that rounds up to 2^(E - 2) included) and
+// E - 1 beyond (the next m above 1.5 gives 1 + 2/3 ulp, which rounds to 1 + ulp); infinity clamps to 127.
 __device__ __forceinline__ int e2m1_exp(float amax) {
     const uint32_t u = __float_as_uint(fmaxf(amax, 1e-30f));
     return u >= 0x7f800000u ? 127 : (int)((u + 0x3fffffu) >> 23) - 129;
@@ -151,9 +151,9 @@ __host__ __device__ __forceinline__ int64_t mx_act_panel_offset(int64_t row, int
 // sign bit set for every negative input.  AF 0: tests/quant_sim.py:75-81 (mxfp8): e = floor(log2(max(amax, 1e-30))) - 8,
 // codes e4m3(clamp(x / 2^e, +-448)) nearest even.  XF32: fp32 input, else bf16.  Rows >= n_rows are skipped.
 // PAN (e4m3 only): q in the panel layout mx_act_panel_offset defines instead of row-major.
-// Memory bounds it (the e2m1 codes' compares beyond 4096 x 13824: 8192 x 17408 bf16 100 -> 86 us with the search in e2m1_mag and
-// no division in e2m1_exp, which four lanes now do where one did).  A thread per block read 64 bytes on its own, one 64-byte line per lane and load, and left a panel
-// chunk's stores to sixteen workgroups; here a wave's loads are contiguous (1 KB of bf16), and a panel workgroup owns
+// Memory bounds it (e2m1 beyond 4096 x 13824: its vector work; 8192 x 17408 bf16 100 -> 86 us with the search in e2m1_mag
+// and no division in e2m1_exp, which four lanes do where a thread per block did one).  A thread per block read 64 bytes on
+// its own, one 64-byte line per lane and load, and left a panel chunk's stores to sixteen workgroups; here a wave's loads are contiguous (1 KB of bf16), and a panel workgroup owns
 // whole 2 KB chunks: 16 rows x 128 inputs, four of them requested at once.
 template <int AF, bool XF32, bool PAN = false, int U = PAN ? 4 : 1>       // U: 8-input pieces per thread
 __global__ __launch_bounds__(256) void mx_quant_act_kernel(const void* __restrict__ x, int64_t ldx,
@@ -164,7 +164,8 @@ __global__ __launch_bounds__(256) void mx_quant_act_kernel(const void* __restric
     const int row = PAN ? blockIdx.y * 16 + (tid >> 4) : blockIdx.y;
     int k[U];                                              // piece u: inputs k[u] .. + 7 (whole 32-input blocks in range)
 #pragma unroll
-    for (int u = 0; u < U; u++) k[u] = PAN ? (blockIdx.x * U + u) * 128 + (tid & 15) * 8 : ((blockIdx.x * U + u) * 256 + tid) * 8;
+    for (int u = 0; u < U; u++)
+        k[u] = PAN ? (blockIdx.x * U + u) * 128 + (tid & 15) * 8 : ((blockIdx.x * U + u) * 256 + tid) * 8;
     float v[U][8];
     const int64_t lrow = min(row, M - 1);                  // loads first, in range; the row count is read under them
 #pragma unroll
@@ -1080,11 +1081,12 @@ static bool mx_mid_fits(int a_fmt, int64_t M, int64_t K) {
     return a_fmt != PRISM_MX_E4M3_PANELS && K <= (1 << 22) && M <= (1 << 16);
 }
 
-// Whether the mid kernel takes the shape by default.  Up to 16 rows: e2m1 batches from 20 M weights (16 x 34816 x 5120 30.1 -> 21.7 us,
-// 5120^2 at 1 / 16 rows 6.2 / 9.2 -> 5.6 / 6.8; 1 x 1024 x 5120 3.8 against 4.7), and of e4m3 the wide ones the split
+// Whether the mid kernel takes the shape by default.  Up to 16 rows: e2m1 batches from 20 M weights (16 x 34816 x 5120 30.1
+// -> 21.7 us, 5120^2 at 1 / 16 rows 6.2 / 9.2 -> 5.6 / 6.8; 1 x 1024 x 5120 3.8 against 4.7), and of e4m3 the wide ones the split
 // decode would take (34816 x 5120 at 1 / 16 rows 26.3 / 25.9 -> 19.9 / 22.9 us; at 5120 x 17408 and 16 rows the split stays
 // ahead, 16.7 against 17.5); with the weights streamed from HBM, as a model's are (already in the caches, the decode
-// kernel is ahead at 1-4 rows: 5120^2 3.9 against 5.3).  Beyond, from 8 M weights (17 x 1024 x 2048 4.1 against 4.6), measured at K = 5120 (both sides go with K): about 3 us and
+// kernel is ahead at 1-4 rows: 5120^2 3.9 against 5.3).  Beyond, from 8 M weights (17 x 1024 x 2048 4.1 against 4.6),
+// measured at K = 5120 (both sides go with K): about 3 us and
 // 5.6 ns (e2m1) or 7.2 ns (e4m3) per 16 x 16 outputs, against the tile kernel's 21 us and 75 ns per 64 x 256 tile up to
 // one per CU, 45 us per round of two beyond (us, mid / tile: e2m1 24 x 34816 28.1 / 27.9, 64 x 13824 21 / 29, 128 x 5120
 // 19.1 / 20.3, 128 x 13824 37 / 28; e4m3 32 x 13824 16 / 27.5, 40 x 5120 10.5 / 22).
@@ -1155,9 +1157,9 @@ extern "C" int prism_mxfp4_quant_act(const void* x, int x_f32, int64_t ldx, cons
         else hipLaunchKernelGGL((mx_quant_act_kernel<0, false, true>), grid, dim3(256), 0, st, x, ldx, inv, q, s,
                                 n_rows, (int)M, (int)K);
     } else if (fmt == PRISM_MX_E4M3) { if (x_f32) QA(0, true); else QA(0, false); }
-    else if (!x_f32 && M > 1024 && K > 16384)              // long batches of long rows: two loads in flight (8192 x 17408 80
+    else if (!x_f32 && M > 1024 && K > 16384)              // long batches of long rows: two loads in flight (8192 x 17408
         hipLaunchKernelGGL((mx_quant_act_kernel<4, false, false, 2>), dim3((unsigned)((K + 4095) / 4096), (unsigned)M),
-                           dim3(256), 0, st, x, ldx, inv, q, s, n_rows, (int)M, (int)K);           // against 86 us)
+                           dim3(256), 0, st, x, ldx, inv, q, s, n_rows, (int)M, (int)K);           // 91 -> 85 us)
     else { if (x_f32) QA(4, true); else QA(4, false); }
 #undef QA
     PRISM_LAUNCH_CHECK();

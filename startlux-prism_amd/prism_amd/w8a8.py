@@ -203,8 +203,8 @@ def workspace(dev, panels=0, stream=None):
     """The workspace of the packed Q8_0 GEMM on dev's current stream (the reference schema's `workspace`, allocated once
     per device as kernels/cuda_ext.py:138-143 does): the "stream" kernel's handoff words, zeroed once and left zeroed by
     every launch, then the prefill's panel copy of the activations.  Under graph capture the words alone, or, for a call
-    that copies `panels` bytes of activations, the room for that alone, and None on a device with no eager call yet (the words' zero fill would be a graph
-    node): "auto" then picks another kernel and "stream" raises.  See scratch.py for what calls may share."""
+    that copies `panels` bytes of activations, the room for that alone, and None on a device with no eager call yet (the
+    words' zero fill would be a graph node): "auto" then picks another kernel and "stream" raises."""
     return _WS.get(dev, not panels, Q8_HANDOFF_BYTES + panels, stream)
 
 
