@@ -96,14 +96,15 @@ def _check_device(dev):
     return idx
 
 
+raw_stream = torch._C._cuda_getCurrentRawStream          # torch's current stream handle on a device index
+
+
 def stream_of(t):
     """torch's current stream handle on t's device."""
-    return raw_stream(_check_device(t.device))
-
-
-def raw_stream(idx):
-    """torch's current stream handle on device idx."""
-    return torch._C._cuda_getCurrentRawStream(idx)
+    dev = t.device
+    if t.is_cuda and dev.index in _checked:
+        return raw_stream(dev.index)
+    return raw_stream(_check_device(dev))
 
 
 def ptr(t):

@@ -29,11 +29,11 @@ SPLIT_WS_BYTES = 32 << 20     # the split decode's segment sums: 1 KB per (1024-
 _WS = scratch.Scratch(SPLIT_WS_BYTES)
 
 
-def split_workspace(dev, need=None, stream=None):
+def split_workspace(dev, need=None):
     """The workspace of the split decode (kernel "split") on dev's current stream: its segment sums, rewritten by every
     launch.  None under graph capture on a device with no eager call yet: "auto" then picks another kernel and "split"
     raises.  need: the bytes a call uses, all that a captured one gets."""
-    return _WS.get(dev, True, need, stream)
+    return _WS.get(dev, True, need)
 
 
 class MX4(NamedTuple):
@@ -204,7 +204,7 @@ def gemm(a_q, a_s, w: MX4, out, n_rows, epi=0, out_stride=None, kernel="auto"):
     ldo = out.stride(0) if out_stride is None else out_stride
     st, ws = L.stream_of(a_q), None
     if fmt == E4M3 and M <= 16 and kernel in ("auto", "split"):
-        ws = split_workspace(a_q.device, max(16, (K + 1023) // 1024 * (N // 16) * 1024), st)
+        ws = _WS.get(a_q.device, True, max(16, (K + 1023) // 1024 * (N // 16) * 1024), st)
     if kernel == "split" and ws is None:
         raise L.PrismError('kernel "split" needs the device workspace, made outside graph capture: run one eager call '
                            'first')

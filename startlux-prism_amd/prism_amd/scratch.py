@@ -41,7 +41,9 @@ class Scratch:
         """The buffer for a call on dev's current stream (stream: its handle, if the caller has it).  zeroed: the call uses
         the zeroed bytes (and no others); need: the bytes the call has a use for, where they are known (all that a captured
         one gets, whose graph's pool keeps them)."""
-        idx = dev.index if dev.index is not None else torch.cuda.current_device()
+        idx = dev.index
+        if idx is None:
+            idx = torch.cuda.current_device()
         if _capturing():
             if idx not in self._captured:
                 return None

@@ -187,7 +187,7 @@ def gemm(xq, a, xs, w: W4, out, n_rows, epi=0, cfg=None, pdl=0, kernel="auto"):
     if Mx != M:
         raise ValueError("xs rows must equal xq rows")
     st = L.stream_of(xq)
-    ws = KW8.workspace(xq.device, 0, st) if M <= 16 and kernel in ("auto", "stream") else None
+    ws = KW8._WS.get(xq.device, True, None, st) if M <= 16 and kernel in ("auto", "stream") else None
     if kernel == "stream" and ws is None:
         raise L.PrismError('kernel "stream" needs the device workspace, made outside graph capture: run one eager '
                            'call first')

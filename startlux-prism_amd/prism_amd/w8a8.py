@@ -199,13 +199,13 @@ Q8_WS_BYTES = Q8_HANDOFF_BYTES + (96 << 20)
 _WS = scratch.Scratch(Q8_WS_BYTES, zeroed=Q8_HANDOFF_BYTES)
 
 
-def workspace(dev, panels=0, stream=None):
+def workspace(dev, panels=0):
     """The workspace of the packed Q8_0 GEMM on dev's current stream (the reference schema's `workspace`, allocated once
     per device as kernels/cuda_ext.py:138-143 does): the "stream" kernel's handoff words, zeroed once and left zeroed by
     every launch, then the prefill's panel copy of the activations.  Under graph capture the words alone, or, for a call
     that copies `panels` bytes of activations, the room for that alone, and None on a device with no eager call yet (the
     words' zero fill would be a graph node): "auto" then picks another kernel and "stream" raises."""
-    return _WS.get(dev, not panels, Q8_HANDOFF_BYTES + panels, stream)
+    return _WS.get(dev, not panels, Q8_HANDOFF_BYTES + panels)
 
 
 def _gemm_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
@@ -225,7 +225,7 @@ def _gemm_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
     pan = pan if Q8_HANDOFF_BYTES + pan <= Q8_WS_BYTES else 0
     st, ws = L.stream_of(a), None
     if pan or (M <= 16 and kernel in ("auto", "decode", "stream")):
-        ws = workspace(a.device, pan, st)
+        ws = _WS.get(a.device, not pan, Q8_HANDOFF_BYTES + pan, st)
     if kernel == "stream" and ws is None and asked == "auto":
         kernel = "auto"             # the table's pick needs the workspace; the library then picks without it
     if kernel == "stream" and ws is None:
@@ -242,12 +242,12 @@ PC_WS_BYTES = 96 << 20        # as the reference's workspace (kernels/cuda_ext.p
 _PCWS = scratch.Scratch(PC_WS_BYTES)
 
 
-def pc_workspace(dev, need=None, stream=None):
+def pc_workspace(dev, need=None):
     """The workspace of the per-channel GEMM on dev's current stream: the split decode's int32 slots (kernel "split") or
     the tile kernel's panel copy of the activations (wide projections from 1024 rows), rewritten by every launch.  None
     under graph capture on a device with no eager call yet: "auto" then picks another kernel and "split" raises.  need: the
     bytes a call can use, all that a captured one gets."""
-    return _PCWS.get(dev, True, need, stream)
+    return _PCWS.get(dev, True, need)
 
 
 _PC_KERNELS = {"auto": -1, "tile": 0, "decode": 1, "split": 2}
@@ -275,7 +275,7 @@ def _gemm_pc_packed(a, a_s, w, out, n_rows, gk, epi, kernel):
     st, ws = L.stream_of(a), None
     if use_ws:
         slots = (12 * M * w.n + 255) // 256 * 256 if M <= 512 else 0
-        ws = pc_workspace(a.device, slots + (M + 15) // 16 * 16 * K, st)
+        ws = _PCWS.get(a.device, True, slots + (M + 15) // 16 * 16 * K, st)
     if kernel == "split" and ws is None and asked == "auto":
         kernel = "auto"             # the table's pick needs the workspace; the library then picks without it
     if kernel == "split" and ws is None:
